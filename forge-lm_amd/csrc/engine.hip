@@ -173,6 +173,7 @@ struct fh_context {
 namespace fh {
 hipStream_t context_stream(fh_context* c) { return c->stream; }
 int context_device(fh_context* c) { return c->device; }
+int context_cus(fh_context* c) { return c->props.multiProcessorCount; }
 OpsState*& context_ops(fh_context* c) { return c->ops; }
 }  // namespace fh
 
@@ -1063,13 +1064,17 @@ int fh_matmul_nn(fh_context* c, const void* a_dev, const void* b_dev, void* y_de
   const float* a = static_cast<const float*>(a_dev);
   float* y = static_cast<float*>(y_dev);
   const float* res = accumulate ? y : nullptr;  // each output element is read, then written, by one lane
-  const bool bf = dtype == FH_DTYPE_BF16;
+  if (dtype == FH_DTYPE_F32) {
+    FH_TRY(fh_op_matmul_nn(c, a_dev, b_dev, y_dev, 1, M, K, N, accumulate));
+    HIP_TRY(hipStreamSynchronize(st));
+    return FH_OK;
+  }
   hipError_t e = hipSuccess;
   if (K % 32 == 0) {
     // the GEMM takes the weights transposed, plus room for split-K partials (or,
     // for bf16 with many rows, for a rounded to bf16: the window path's kernel)
-    const bool big = bf && M >= 256 && K % 64 == 0;
-    const size_t esz = bf ? 2 : 4, part_floats = big ? 0 : (size_t)8 * M * N;
+    const bool big = M >= 256 && K % 64 == 0;
+    const size_t esz = 2, part_floats = big ? 0 : (size_t)8 * M * N;
     // an accumulating bf16 product may split K in two: first halves' sums and tile counters
     const size_t ws_floats = big && res ? (size_t)M * N : 0;
     const int ncnt = big && res ? ((M + 255) / 256) * ((N + 255) / 256) : 0;
@@ -1089,16 +1094,11 @@ int fh_matmul_nn(fh_context* c, const void* a_dev, const void* b_dev, void* y_de
       if (e == hipSuccess)
         e = res ? launch_gemm_bf16_split(st, ah, M, K, wt, N, nullptr, res, y, ws, ws_floats, cnt, ncnt)
                 : launch_gemm_bf16(st, ah, M, K, wt, N, nullptr, EPI_NONE, res, y, nullptr);
-    } else if (bf) {
+    } else {
       e = launch_transpose<bf16_t>(st, static_cast<const bf16_t*>(b_dev), K, N, reinterpret_cast<bf16_t*>(tmp));
       if (e == hipSuccess)
         e = launch_gemm_mfma<bf16_t>(st, a, M, K, reinterpret_cast<const bf16_t*>(tmp), N, nullptr, EPI_NONE, res, y,
                                      part, part_floats, c->props.multiProcessorCount);
-    } else {
-      e = launch_transpose<float>(st, static_cast<const float*>(b_dev), K, N, reinterpret_cast<float*>(tmp));
-      if (e == hipSuccess)
-        e = launch_gemm_mfma<float>(st, a, M, K, reinterpret_cast<const float*>(tmp), N, nullptr, EPI_NONE, res, y,
-                                    part, part_floats, c->props.multiProcessorCount);
     }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     int split_err = 0;
@@ -1109,8 +1109,7 @@ int fh_matmul_nn(fh_context* c, const void* a_dev, const void* b_dev, void* y_de
                      (split_err & 1) ? "the wait for the first half exceeded its bound"
                                      : "the halves ran on different XCDs");
   } else {
-    e = bf ? launch_gemm<bf16_t>(st, a, M, K, static_cast<const bf16_t*>(b_dev), N, nullptr, EPI_NONE, res, y)
-           : launch_gemm<float>(st, a, M, K, static_cast<const float*>(b_dev), N, nullptr, EPI_NONE, res, y);
+    e = launch_gemm<bf16_t>(st, a, M, K, static_cast<const bf16_t*>(b_dev), N, nullptr, EPI_NONE, res, y);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
   }
   HIP_TRY(e);

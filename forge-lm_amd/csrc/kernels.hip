@@ -300,9 +300,16 @@ __global__ __launch_bounds__(256) void k_splitk_epilogue(const float* __restrict
   // the bias and residual are requested with the partials (one round trip, not three)
   const float bn = bias ? bias[n] : 0.f, rn = res ? res[idx] : 0.f;
   float s = 0.f;
-  // partials summed in order; the unrolled loads of a batch are independent and go out together
-#pragma unroll 8
-  for (int i = 0; i < S; i++) s += part[(size_t)i * M * N + idx];
+  // partials summed in order; the loads of a batch of 8 (the last one's again past S) go out
+  // together: one at a time, 3 splits cost three round trips
+  for (int i0 = 0; i0 < S; i0 += 8) {
+    float t[8];
+#pragma unroll
+    for (int ii = 0; ii < 8; ii++) t[ii] = part[(size_t)min(i0 + ii, S - 1) * M * N + idx];
+#pragma unroll
+    for (int ii = 0; ii < 8; ii++)
+      if (i0 + ii < S) s += t[ii];
+  }
   if (bias) s += bn;
   if (epi == EPI_GELU) s = gelu_tanh(s);
   if (res) s += rn;

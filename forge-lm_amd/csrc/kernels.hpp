@@ -185,6 +185,21 @@ bool gemm_skinny_fits(int M, int K, int N);
 hipError_t launch_gemm_skinny(hipStream_t st, const float* x, int M, int K, const float* Wt, int N,
                               const float* bias, int epi, float* y, int* splits);
 
+// fp32 products on the bf16 matrix cores (gemm_split.hip), operands read in place: y[s] =
+// epi(op(a[s]) @ op(b[s]) + bias) (+ res) for s < slots.  mode 0 NN (a [M,K], b [K,N]), 1 NT
+// (b [N,K]), 2 TN (a [K,M]); gelu and res exclude each other; res may be y (accumulation).
+// part (may be null) has room for part_floats of K-split partial sums.
+// gemm_split_fits: sizes whose offsets and grid are in range.
+// gemm_split_part_floats: what the product would use of at most `most` floats.
+bool gemm_split_fits(int slots, int M, int K, int N);
+size_t gemm_split_part_floats(int slots, int M, int K, int N, size_t most, int cus);
+hipError_t launch_gemm_split(hipStream_t st, int mode, const float* a, const float* b, int slots, int M, int K, int N,
+                             const float* bias, int gelu, const float* res, float* y, float* part,
+                             size_t part_floats, int cus);
+// a [M,K] @ b [N,K]^T as partial sums part[*splits][M][N] (at least one) for a fused epilogue.
+hipError_t launch_gemm_split_parts(hipStream_t st, const float* a, const float* b, int M, int K, int N, float* part,
+                                   size_t part_floats, int cus, int* splits);
+
 // Wt[n][k] = W[k][n].
 template <typename WT>
 hipError_t launch_transpose(hipStream_t st, const WT* W, int K, int N, WT* Wt);

@@ -12,8 +12,8 @@
 //
 // The kernels are the straightforward HBM-bound forms: grid-stride elementwise
 // loops, one block per row for the row reductions, column sums in fixed
-// row-chunk order, a 64x64 LDS-tiled FMA kernel for the (batched) matmuls with
-// the large plain NN product on the MFMA GEMM.  Results follow CpuBackend
+// row-chunk order; the (batched) matmuls run on the split GEMM (gemm_split.hip).
+// Results follow CpuBackend
 // within the reference's own GPU-contract tolerances (GpuBackendTests.cs:23-24:
 // 1e-4 forward, 1e-2 backward); the gathers, copies, masks and the embedding
 // scatter-add (which adds each index's rows in ascending position, as the CPU
@@ -34,6 +34,7 @@ namespace fh {
 int set_error(int code, const char* msg);
 hipStream_t context_stream(fh_context* c);
 int context_device(fh_context* c);
+int context_cus(fh_context* c);
 struct OpsState;
 OpsState*& context_ops(fh_context* c);
 
@@ -63,6 +64,7 @@ __device__ __forceinline__ float ops_block_max(float v, float* red) {
 unsigned grid_for(size_t n) { return (unsigned)std::min<size_t>((n + kT - 1) / kT, 65536); }
 
 // ---- matmuls: y[s] (+)= op(a[s]) @ op(b[s]), 64x64 tiles, k steps of 16 ------------
+// for sizes that the split GEMM does not take (gemm_split_fits), with 64-bit offsets
 // MODE 0 NN (a [M,K], b [K,N]), 1 NT (b [N,K]), 2 TN (a [K,M]).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, const float* __restrict__ b,
@@ -545,13 +547,25 @@ int upload_ints(fh_context* c, OpsState* o, const int32_t* host, size_t n, int**
   return FH_OK;
 }
 
+// the partial sums of a split K take at most this much of the context's scratch (64 MB)
+constexpr size_t kSplitPartFloats = (size_t)16 << 20;
+
 int matmul_common(fh_context* c, int mode, const void* a, const void* b, void* y, int slots, int M, int K, int N,
                   int acc) {
   OPS_PROLOGUE(c);
   OPS_ARG(a && b && y, "null buffer");
   OPS_ARG(slots > 0 && slots <= 65535 && M > 0 && K > 0 && N > 0, "slots (at most 65535), M, K and N must be positive");
-  if (mode == 0 && slots == 1 && K % 32 == 0 && (size_t)M * K * N >= ((size_t)1 << 24))
-    return fh_matmul_nn(c, a, b, y, M, K, N, FH_DTYPE_F32, acc);  // the MFMA GEMM
+  if (gemm_split_fits(slots, M, K, N)) {
+    const int cus = context_cus(c);
+    const size_t pf = gemm_split_part_floats(slots, M, K, N, kSplitPartFloats, cus);
+    void* part = nullptr;
+    if (pf) FH_TRY(ops_scratch(c, ops_, pf * sizeof(float), &part));
+    HIP_TRY(launch_gemm_split(st_, mode, static_cast<const float*>(a), static_cast<const float*>(b), slots, M, K, N,
+                              nullptr, 0, acc ? static_cast<const float*>(y) : nullptr, static_cast<float*>(y),
+                              static_cast<float*>(part), pf, cus));
+    return FH_OK;
+  }
+  // sizes past the split GEMM's 32-bit offsets
   dim3 grid((N + 63) / 64, (M + 63) / 64, slots);
   const float* fa = static_cast<const float*>(a);
   const float* fb = static_cast<const float*>(b);

@@ -122,8 +122,9 @@ int fh_buffer_checksum(fh_context* ctx, const void* src_dev, size_t bytes, uint6
 
 /* ITensorBackend.MatMulNN(a, b, y, M, K, N, accumulate) (ITensorBackend.cs:22) on
  * device buffers: y[M][N] = a[M][K] @ b[K][N], or += when accumulate != 0.  a and
- * y fp32; b fp32 or bf16 (dtype).  The product runs on the MFMA GEMM the token
- * loop uses for more than 4 rows (bf16: a rounded to bf16, fp32 accumulation).
+ * y fp32; b fp32 or bf16 (dtype).  fp32: the product of fh_op_matmul_nn; bf16: the
+ * MFMA GEMM the token loop uses for more than 4 rows (a rounded to bf16, fp32
+ * accumulation).
  * Synchronous. */
 int fh_matmul_nn(fh_context* ctx, const void* a_dev, const void* b_dev, void* y_dev, int M, int K, int N,
                  int dtype, int accumulate);

@@ -367,6 +367,62 @@ def test_matmul_matches_cpu(fhp, oracle, tb):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("slots,M,K,N", [(1, 1, 1, 1), (2, 64, 32, 64), (3, 65, 33, 63), (1, 129, 31, 257),
+                                         (5, 40, 331, 64), (1, 300, 2049, 130), (1, 1025, 768, 1100),
+                                         (2, 200, 4096, 96)])
+def test_split_matmul_tiles_and_remainders(fhp, tb, mode, slots, M, K, N):
+    """Products around the split GEMM's tiles (64 and 128 rows and columns, 32 k), whole and split
+    over K, plain and accumulated, against float64.  fp32 sums of K products round by 2^-24 K^0.5
+    of their own size in the 2-norm; the split's left-out terms (2^-26 each) stay below that."""
+    g = np.random.default_rng(slots * 1000 + M + K + N)
+    a = g.standard_normal((slots, K, M) if mode == "tn" else (slots, M, K)).astype(np.float32)
+    b = g.standard_normal((slots, N, K) if mode == "nt" else (slots, K, N)).astype(np.float32)
+    prior = g.standard_normal((slots, M, N)).astype(np.float32)
+    A = a.astype(np.float64).transpose(0, 2, 1) if mode == "tn" else a.astype(np.float64)
+    B = b.astype(np.float64).transpose(0, 2, 1) if mode == "nt" else b.astype(np.float64)
+    want = A @ B
+    fn = {"nn": tb.BatchedMatMulNN, "nt": tb.BatchedMatMulNT, "tn": tb.BatchedMatMulTN}[mode]
+    for acc in (False, True):
+        y = dup(fhp, prior, slots * M, N)
+        fn(dup(fhp, a, slots * a.shape[1], a.shape[2]), dup(fhp, b, slots * b.shape[1], b.shape[2]), y, slots, M, K, N,
+           acc)
+        tb.EnsureHostCurrent(y)
+        err = y.Data.reshape(want.shape) - want - (prior if acc else 0)
+        size = np.linalg.norm(want) + (np.linalg.norm(prior) if acc else 0)
+        assert np.linalg.norm(err) <= 2.0 ** -24 * (2 + np.sqrt(K)) * size, np.linalg.norm(err) / size
+
+
+@pytest.mark.gpu
+def test_split_matmul_infinities_and_nan(fhp, tb):
+    """Infinite, NaN and overflowing sums are those of fp32 arithmetic; other outputs stay exact to fp32."""
+    g = np.random.default_rng(5)
+    M, K, N = 150, 96, 140
+    a = g.standard_normal((M, K)).astype(np.float32)
+    b = g.standard_normal((K, N)).astype(np.float32)
+    b[7] = 1.0  # exactly representable in bf16: its lower parts are zero
+    a[3, 7] = np.inf
+    a[5, 7], a[5, 8] = np.inf, -np.inf
+    b[8] = 2.0
+    a[9, 2] = np.nan
+    a[11, :] = 0.0
+    a[11, 20], b[20, 4] = 3.4e38, 3.0  # overflows
+    a[12, 21], b[21, :] = 3.4028235e38, 0.5  # rounds to infinity in bf16, is finite in fp32
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
+    y = fhp.Tensor(M, N)
+    tb.MatMulNN(dup(fhp, a, M, K), dup(fhp, b, K, N), y, M, K, N)
+    tb.EnsureHostCurrent(y)
+    got = y.Data.reshape(M, N)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    np.testing.assert_array_equal(got[inf], want[inf])
+    ok = np.isfinite(want)
+    assert np.all(np.isfinite(got[ok]))
+    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.gpu
 def test_elementwise_matches_cpu(fhp, oracle, tb):
     # GpuBackendTests.Elementwise_MatchesCpu
     rng = NetRng(oracle, 102)
