@@ -11,8 +11,8 @@
 // mirror, which owns the device copies of its tensors.
 //
 // The kernels are the straightforward HBM-bound forms: grid-stride elementwise
-// loops, one block per row for the row reductions, column sums in fixed
-// row-chunk order; the (batched) matmuls run on the split GEMM (gemm_split.hip).
+// loops, one block or wave per row for the row reductions, column sums in chunks of rows
+// in a fixed order; the (batched) matmuls run on the split GEMM (gemm_split.hip).
 // Results follow CpuBackend
 // within the reference's own GPU-contract tolerances (GpuBackendTests.cs:23-24:
 // 1e-4 forward, 1e-2 backward); the gathers, copies, masks and the embedding
@@ -59,6 +59,17 @@ __device__ __forceinline__ float ops_block_max(float v, float* red) {
   if (lane == 0) red[w] = v;
   __syncthreads();
   return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// sum over a block of 256 in double (red: 256)
+__device__ __forceinline__ double block_sum_double(double s, double* red) {
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+    __syncthreads();
+  }
+  return red[0];
 }
 
 unsigned grid_for(size_t n) { return (unsigned)std::min<size_t>((n + kT - 1) / kT, 65536); }
@@ -181,45 +192,69 @@ __global__ __launch_bounds__(256) void k_transpose_f32(const float* __restrict__
     if (c0 + i < cols && r0 + tx < rows) out[(size_t)(c0 + i) * rows + r0 + tx] = tile[tx][i];
 }
 
-// Column sums over a chunk of rows: sums[chunk][c] = sum of rows in the chunk, in
-// row order.  With one chunk the kernel adds straight into dst (dst[c] + rows in
-// order, the CPU's sequence); otherwise k_sum_chunks adds the chunks in order.
-constexpr int kRowChunk = 256;
-// KIND 0: plain column sums of y (SumRows).  KIND 1: LayerNorm's dW and dB
-// (sums of dOut * xhat and of dOut) into dst and dst2.
-template <int KIND>
-__global__ void k_col_sums(const float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ mean,
-                           const float* __restrict__ rstd, int rows, int cols, float* __restrict__ dst,
-                           float* __restrict__ dst2, float* __restrict__ part, int chunks) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  const int r0 = blockIdx.y * kRowChunk, r1 = min(rows, r0 + kRowChunk);
-  float s = chunks == 1 ? dst[c] : 0.f;
-  float s2 = (KIND == 1 && chunks == 1) ? dst2[c] : 0.f;
-  for (int r = r0; r < r1; r++) {
-    const float d = y[(size_t)r * cols + c];
-    if (KIND == 1) {
-      const float xhat = (x[(size_t)r * cols + c] - mean[r]) * rstd[r];
-      s = s + d * xhat;
-      s2 = s2 + d;
-    } else {
-      s = s + d;
+// Column sums, HBM-bound: a block of four waves takes 64 columns of a chunk of rows, a
+// lane one column; wave w adds rows w, w + 4, ... in order with 8 loads in flight, and the
+// waves' sums add up in wave order.  The chunks are small enough to give every CU several
+// blocks (2048 x 3072: one 256-row chunk per block and one load at a time took 60 us, this
+// and the chunks' sum 10).  With one chunk the sums go straight into dst (dst[c] + sum),
+// otherwise into part[chunk][c] for k_sum_chunks.
+constexpr int kSumWaves = 4;
+__global__ __launch_bounds__(64 * kSumWaves) void k_col_sums(const float* __restrict__ y, int rows, int cols,
+                                                             int chunk_rows, float* __restrict__ dst,
+                                                             float* __restrict__ part) {
+  __shared__ float red[kSumWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = blockIdx.x * 64 + lane;
+  const int r0 = blockIdx.y * chunk_rows, r1 = min(rows, r0 + chunk_rows);
+  float s = 0.f;
+  if (c < cols) {
+    int r = r0 + w;
+    for (; r + 7 * kSumWaves < r1; r += 8 * kSumWaves) {
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) t[i] = y[(size_t)(r + i * kSumWaves) * cols + c];
+#pragma unroll
+      for (int i = 0; i < 8; i++) s += t[i];
     }
+    for (; r < r1; r += kSumWaves) s += y[(size_t)r * cols + c];
   }
-  if (chunks == 1) {
-    dst[c] = s;
-    if (KIND == 1) dst2[c] = s2;
-  } else {
+  red[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || c >= cols) return;
+  for (int i = 1; i < kSumWaves; i++) s += red[i][lane];
+  if (part)
     part[(size_t)blockIdx.y * cols + c] = s;
-    if (KIND == 1) part[((size_t)chunks + blockIdx.y) * cols + c] = s2;
-  }
+  else
+    dst[c] = dst[c] + s;
 }
 
-__global__ void k_sum_chunks(const float* __restrict__ part, int chunks, int cols, float* __restrict__ dst) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
+// dst[k][c] += the sum of the chunks' part[chunk][k][c] for k < gridDim.y (dst0, dst1): 16
+// waves take every 16th chunk each, 8 loads in flight, and add up in wave order.
+constexpr int kChunkWaves = 16;
+__global__ __launch_bounds__(64 * kChunkWaves) void k_sum_chunks(const float* __restrict__ part, int chunks, int cols,
+                                                                 float* __restrict__ dst0, float* __restrict__ dst1) {
+  __shared__ float red[kChunkWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int c = blockIdx.x * 64 + lane;
+  const size_t ld = (size_t)gridDim.y * cols;
   float s = 0.f;
-  for (int k = 0; k < chunks; k++) s = s + part[(size_t)k * cols + c];
+  if (c < cols) {
+    const float* p = part + (size_t)blockIdx.y * cols + c;
+    int k = w;
+    for (; k + 7 * kChunkWaves < chunks; k += 8 * kChunkWaves) {
+      float t[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) t[i] = p[(size_t)(k + i * kChunkWaves) * ld];
+#pragma unroll
+      for (int i = 0; i < 8; i++) s += t[i];
+    }
+    for (; k < chunks; k += kChunkWaves) s += p[(size_t)k * ld];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || c >= cols) return;
+  for (int i = 1; i < kChunkWaves; i++) s += red[i][lane];
+  float* dst = blockIdx.y ? dst1 : dst0;
   dst[c] = dst[c] + s;
 }
 
@@ -247,6 +282,69 @@ __global__ __launch_bounds__(256) void k_ln_forward(const float* __restrict__ x,
   for (int c = threadIdx.x; c < cols; c += 256) out[(size_t)r * cols + c] = (xr[c] - mu) * rs * w[c] + b[c];
 }
 
+// dx of every row and the column sums of dOut * xhat and dOut, reading dOut and x once: a
+// wave keeps its row in registers (lane l: columns l, l + 64, ...; cols <= 64 VPL) and adds
+// its rows' terms up per column; the block's waves add up in wave order into
+// part[block][2][cols] (HBM-bound; 2048 x 768: 6 + 72 + 8 us for dx, the two column sums and
+// their chunks, 8 + 4 this way).
+template <int VPL>
+__global__ __launch_bounds__(256) void k_ln_backward_rows(const float* __restrict__ dout, const float* __restrict__ x,
+                                                          const float* __restrict__ w, const float* __restrict__ mean,
+                                                          const float* __restrict__ rstd, float* __restrict__ dx,
+                                                          int rows, int cols, int rows_per_block,
+                                                          float* __restrict__ part) {
+  __shared__ float red[4][64 * VPL];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int r0 = blockIdx.x * rows_per_block, r1 = min(rows, r0 + rows_per_block);
+  const float inv_n = 1.f / (float)cols;
+  float wc[VPL], sw[VPL], sb[VPL];
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    const int c = lane + 64 * i;
+    wc[i] = c < cols ? w[c] : 0.f;
+    sw[i] = sb[i] = 0.f;
+  }
+  for (int r = r0 + wv; r < r1; r += 4) {
+    const float* dr = dout + (size_t)r * cols;
+    const float* xr = x + (size_t)r * cols;
+    const float mu = mean[r], rs = rstd[r];
+    float d[VPL], xh[VPL];
+#pragma unroll
+    for (int i = 0; i < VPL; i++) {
+      const int c = lane + 64 * i;
+      d[i] = c < cols ? dr[c] : 0.f;
+      xh[i] = c < cols ? xr[c] : 0.f;
+    }
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < VPL; i++) {
+      if (lane + 64 * i >= cols) continue;
+      xh[i] = (xh[i] - mu) * rs;
+      const float dxh = d[i] * wc[i];
+      s1 += dxh;
+      s2 += dxh * xh[i];
+      sw[i] += d[i] * xh[i];
+      sb[i] += d[i];
+    }
+    const float m1 = wave_sum_dpp(s1) * inv_n, m2 = wave_sum_dpp(s2) * inv_n;
+#pragma unroll
+    for (int i = 0; i < VPL; i++) {
+      const int c = lane + 64 * i;
+      if (c < cols) dx[(size_t)r * cols + c] = rs * (d[i] * wc[i] - m1 - xh[i] * m2);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < VPL; i++) red[wv][lane + 64 * i] = k ? sb[i] : sw[i];
+    __syncthreads();
+    for (int c = threadIdx.x; c < cols; c += 256)
+      part[((size_t)blockIdx.x * 2 + k) * cols + c] = red[0][c] + red[1][c] + red[2][c] + red[3][c];
+  }
+}
+
+// rows wider than the registers of a wave: dx by a block per row, the columns by chunks
 __global__ __launch_bounds__(256) void k_ln_backward_dx(const float* __restrict__ dout, const float* __restrict__ x,
                                                         const float* __restrict__ w, const float* __restrict__ mean,
                                                         const float* __restrict__ rstd, float* __restrict__ dx,
@@ -269,6 +367,23 @@ __global__ __launch_bounds__(256) void k_ln_backward_dx(const float* __restrict_
     const float xhat = (xr[c] - mu) * rs, dxhat = dr[c] * w[c];
     dx[(size_t)r * cols + c] = rs * (dxhat - m1 - xhat * m2);
   }
+}
+
+__global__ void k_ln_backward_cols(const float* __restrict__ dout, const float* __restrict__ x,
+                                   const float* __restrict__ mean, const float* __restrict__ rstd, int rows, int cols,
+                                   int chunk_rows, float* __restrict__ part) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= cols) return;
+  const int r0 = blockIdx.y * chunk_rows, r1 = min(rows, r0 + chunk_rows);
+  float s = 0.f, s2 = 0.f;
+#pragma unroll 4
+  for (int r = r0; r < r1; r++) {
+    const float d = dout[(size_t)r * cols + c];
+    s += d * ((x[(size_t)r * cols + c] - mean[r]) * rstd[r]);
+    s2 += d;
+  }
+  part[((size_t)blockIdx.y * 2) * cols + c] = s;
+  part[((size_t)blockIdx.y * 2 + 1) * cols + c] = s2;
 }
 
 // ---- softmax (CpuBackend.cs:446-473; ITensorBackend.cs:117-130) ----------------------
@@ -380,12 +495,13 @@ __global__ __launch_bounds__(256) void k_ce_forward(const float* logits, const i
   if (threadIdx.x == 0) nll[t] = ignored ? 0.f : logf(sum) + mx - tl;
 }
 
-// acc (double, device) += sum of the T per-position terms, in position order
-__global__ void k_ce_accumulate(const float* __restrict__ nll, int T, double* __restrict__ acc) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  float s = 0.f;
-  for (int t = 0; t < T; t++) s = s + nll[t];
-  acc[0] += (double)s;
+// acc (double, device) += sum of the T per-position terms, by one block in double (fixed order)
+__global__ __launch_bounds__(256) void k_ce_accumulate(const float* __restrict__ nll, int T, double* __restrict__ acc) {
+  __shared__ double red[256];
+  double s = 0;
+  for (int t = threadIdx.x; t < T; t += 256) s += (double)nll[t];
+  s = block_sum_double(s, red);
+  if (threadIdx.x == 0) acc[0] += s;
 }
 
 __global__ void k_ce_backward(const float* probs, const int* __restrict__ targets, float* dl, int V, int ignore,
@@ -403,27 +519,46 @@ __global__ void k_ce_backward(const float* probs, const int* __restrict__ target
 }
 
 // ---- sums of squares and AdamW (ITensorBackend.cs:214-265) ---------------------------------
-// per-block double partials of sum x^2; the final pass adds the partials in order
-__global__ __launch_bounds__(256) void k_sumsq_partials(const float* __restrict__ x, size_t n,
-                                                        double* __restrict__ part) {
+// Sum x^2 of up to kSumsqTensors tensors in one launch: block j of a tensor's blocks adds
+// elements j, j + its blocks, ... (in strides of 256) in double, the block's threads add up
+// in a fixed tree, and k_sum_doubles adds the blocks' sums.  HBM-bound; a launch per tensor
+// and a sum by one thread took 141 + 94 us for 20.5M elements in 16 tensors.
+constexpr int kSumsqTensors = 64;
+constexpr int kSumsqPerBlock = 8192;  // elements that a tensor gets a block for, up to kSumsqBlocks
+constexpr int kSumsqBlocks = 512;
+struct SumsqList {
+  const float* x[kSumsqTensors];
+  long long n[kSumsqTensors];
+  int first[kSumsqTensors + 1];  // first block of each tensor
+  int count;
+};
+__global__ __launch_bounds__(256) void k_sumsq(SumsqList l, double* __restrict__ part) {
   __shared__ double red[256];
+  int t = 0;
+  while (t + 1 < l.count && (int)blockIdx.x >= l.first[t + 1]) t++;
+  const float* x = l.x[t];
+  const size_t n = (size_t)l.n[t], step = (size_t)(l.first[t + 1] - l.first[t]) * 256;
   double s = 0;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    s += (double)x[i] * x[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+  size_t i = (size_t)(blockIdx.x - l.first[t]) * 256 + threadIdx.x;
+  for (; i + 7 * step < n; i += 8 * step) {
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = x[i + k * step];
+#pragma unroll
+    for (int k = 0; k < 8; k++) s += (double)v[k] * v[k];
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+  for (; i < n; i += step) s += (double)x[i] * x[i];
+  s = block_sum_double(s, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ void k_sum_doubles(const double* __restrict__ part, int n, double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// out[0] = sum of part[0 .. n) by one block (fixed order)
+__global__ __launch_bounds__(256) void k_sum_doubles(const double* __restrict__ part, int n, double* __restrict__ out) {
+  __shared__ double red[256];
   double s = 0;
-  for (int i = 0; i < n; i++) s += part[i];
-  out[0] = s;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+  s = block_sum_double(s, red);
+  if (threadIdx.x == 0) out[0] = s;
 }
 
 __global__ void k_adamw(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
@@ -587,13 +722,6 @@ int softmax_common(fh_context* c, void* x, int rows, int cols, float scale, int 
   return op_launched("softmax");
 }
 
-int sumsq_partials(hipStream_t st, const float* x, size_t n, double* part, int* blocks) {
-  const int nb = (int)std::min<size_t>(256, std::max<size_t>(1, (n + 255) / 256));
-  hipLaunchKernelGGL(k_sumsq_partials, dim3(nb), dim3(256), 0, st, x, n, part);
-  *blocks = nb;
-  return op_launched("sum of squares");
-}
-
 }  // namespace
 
 extern "C" {
@@ -646,19 +774,22 @@ int fh_op_add_bias(fh_context* c, void* y, const void* bias, int rows, int cols)
 int fh_op_sum_rows(fh_context* c, const void* dy, void* dbias, int rows, int cols) {
   OPS_PROLOGUE(c);
   OPS_ARG(dy && dbias && rows > 0 && cols > 0, "bad arguments");
-  const int chunks = (rows + kRowChunk - 1) / kRowChunk;
+  // chunks of at least 32 rows (64 when that is all of them) until there are about 1024 blocks
+  const int strips = (cols + 63) / 64;
+  const int want = std::max(1, std::min((rows + 31) / 32, (1024 + strips - 1) / strips));
+  const int chunk_rows = rows <= 64 ? rows : (rows + want - 1) / want;
+  const int chunks = (rows + chunk_rows - 1) / chunk_rows;
   float* part = nullptr;
   if (chunks > 1) {
     void* p = nullptr;
     FH_TRY(ops_scratch(c, ops_, (size_t)chunks * cols * sizeof(float), &p));
     part = static_cast<float*>(p);
   }
-  hipLaunchKernelGGL(k_col_sums<0>, dim3((cols + 255) / 256, chunks), dim3(256), 0, st_,
-                     static_cast<const float*>(dy), nullptr, nullptr, nullptr, rows, cols, static_cast<float*>(dbias),
-                     nullptr, part, chunks);
+  hipLaunchKernelGGL(k_col_sums, dim3(strips, chunks), dim3(64 * kSumWaves), 0, st_, static_cast<const float*>(dy),
+                     rows, cols, chunk_rows, static_cast<float*>(dbias), part);
   if (chunks > 1)
-    hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 255) / 256), dim3(256), 0, st_, part, chunks, cols,
-                       static_cast<float*>(dbias));
+    hipLaunchKernelGGL(k_sum_chunks, dim3(strips), dim3(64 * kChunkWaves), 0, st_, part, chunks, cols,
+                       static_cast<float*>(dbias), nullptr);
   return op_launched("sum rows");
 }
 
@@ -721,23 +852,36 @@ int fh_op_layernorm_backward(fh_context* c, const void* dout, const void* x, con
   OPS_ARG(dout && x && w && mean && rstd && dx && dw && db && rows > 0 && cols > 0, "bad arguments");
   const float *fd = static_cast<const float*>(dout), *fx = static_cast<const float*>(x);
   const float *fm = static_cast<const float*>(mean), *fr = static_cast<const float*>(rstd);
-  hipLaunchKernelGGL(k_ln_backward_dx, dim3(rows), dim3(256), 0, st_, fd, fx, static_cast<const float*>(w), fm, fr,
-                     static_cast<float*>(dx), cols);
-  const int chunks = (rows + kRowChunk - 1) / kRowChunk;
-  float* part = nullptr;
-  if (chunks > 1) {
-    void* p = nullptr;
-    FH_TRY(ops_scratch(c, ops_, (size_t)2 * chunks * cols * sizeof(float), &p));
-    part = static_cast<float*>(p);
+  // part[chunk][2][cols] of dW and dB: four rows a block (one a wave), more past 512 blocks
+  const bool wide = cols > 1024;
+  const int per = wide ? std::max(32, (rows + 127) / 128) : std::max(4, ((rows + 511) / 512 + 3) / 4 * 4);
+  const int chunks = (rows + per - 1) / per;
+  void* p = nullptr;
+  FH_TRY(ops_scratch(c, ops_, (size_t)2 * chunks * cols * sizeof(float), &p));
+  float* part = static_cast<float*>(p);
+  const float* fw = static_cast<const float*>(w);
+  float* fdx = static_cast<float*>(dx);
+  if (wide) {
+    hipLaunchKernelGGL(k_ln_backward_dx, dim3(rows), dim3(256), 0, st_, fd, fx, fw, fm, fr, fdx, cols);
+    hipLaunchKernelGGL(k_ln_backward_cols, dim3((cols + 255) / 256, chunks), dim3(256), 0, st_, fd, fx, fm, fr, rows,
+                       cols, per, part);
+  } else {
+#define LN_ROWS(V) \
+  hipLaunchKernelGGL(k_ln_backward_rows<V>, dim3(chunks), dim3(256), 0, st_, fd, fx, fw, fm, fr, fdx, rows, cols, per, part)
+    if (cols <= 64)
+      LN_ROWS(1);
+    else if (cols <= 256)
+      LN_ROWS(4);
+    else if (cols <= 512)
+      LN_ROWS(8);
+    else if (cols <= 768)
+      LN_ROWS(12);
+    else
+      LN_ROWS(16);
+#undef LN_ROWS
   }
-  hipLaunchKernelGGL(k_col_sums<1>, dim3((cols + 255) / 256, chunks), dim3(256), 0, st_, fd, fx, fm, fr, rows, cols,
-                     static_cast<float*>(dw), static_cast<float*>(db), part, chunks);
-  if (chunks > 1) {
-    hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 255) / 256), dim3(256), 0, st_, part, chunks, cols,
-                       static_cast<float*>(dw));
-    hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 255) / 256), dim3(256), 0, st_, part + (size_t)chunks * cols, chunks,
-                       cols, static_cast<float*>(db));
-  }
+  hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 63) / 64, 2), dim3(64 * kChunkWaves), 0, st_, part, chunks, cols,
+                     static_cast<float*>(dw), static_cast<float*>(db));
   return op_launched("layernorm backward");
 }
 
@@ -847,7 +991,7 @@ int fh_op_cross_entropy_forward(fh_context* c, const void* logits, const int32_t
   FH_TRY(op_launched("cross-entropy forward"));
   if (ops_->accumulating) {
     // the loss stays on the device until the accumulation ends (ITensorBackend.cs:154-161)
-    hipLaunchKernelGGL(k_ce_accumulate, dim3(1), dim3(64), 0, st_, nll, T, ops_->acc);
+    hipLaunchKernelGGL(k_ce_accumulate, dim3(1), dim3(256), 0, st_, nll, T, ops_->acc);
     ops_->accumulated_targets += count;
     *loss = 0.f;
     return op_launched("loss accumulation");
@@ -925,18 +1069,31 @@ int fh_op_global_sum_squares(fh_context* c, const void* const* xs, const int64_t
   *out = 0;
   if (count == 0) return FH_OK;
   for (int i = 0; i < count; i++) OPS_ARG(xs[i] && ns[i] >= 0, "bad tensor %d", i);
+  auto blocks_of = [](int64_t n) {
+    return (int)std::min<int64_t>(kSumsqBlocks, (n + kSumsqPerBlock - 1) / kSumsqPerBlock);
+  };
+  size_t blocks = 0;
+  for (int i = 0; i < count; i++) blocks += blocks_of(ns[i]);
   void* p = nullptr;
-  FH_TRY(ops_scratch(c, ops_, ((size_t)count * 256 + 1) * sizeof(double), &p));
-  double* part = static_cast<double*>(p);
-  int off = 0;
-  for (int i = 0; i < count; i++) {
-    if (ns[i] == 0) continue;
+  FH_TRY(ops_scratch(c, ops_, (blocks + 1) * sizeof(double), &p));
+  double* res = static_cast<double*>(p);
+  double* part = res + 1;
+  size_t off = 0;
+  for (int i = 0; i < count;) {
+    SumsqList l{};
     int nb = 0;
-    FH_TRY(sumsq_partials(st_, static_cast<const float*>(xs[i]), (size_t)ns[i], part + off, &nb));
+    for (; i < count && l.count < kSumsqTensors; i++) {
+      if (ns[i] == 0) continue;
+      l.x[l.count] = static_cast<const float*>(xs[i]);
+      l.n[l.count] = ns[i];
+      l.first[l.count++] = nb;
+      nb += blocks_of(ns[i]);
+    }
+    l.first[l.count] = nb;
+    if (nb) hipLaunchKernelGGL(k_sumsq, dim3(nb), dim3(256), 0, st_, l, part + off);
     off += nb;
   }
-  double* res = part + (size_t)count * 256;
-  hipLaunchKernelGGL(k_sum_doubles, dim3(1), dim3(64), 0, st_, part, off, res);
+  hipLaunchKernelGGL(k_sum_doubles, dim3(1), dim3(256), 0, st_, part, (int)off, res);
   FH_TRY(op_launched("sum of squares"));
   HIP_TRY(hipMemcpyAsync(out, res, sizeof(double), hipMemcpyDeviceToHost, st_));
   HIP_TRY(hipStreamSynchronize(st_));

@@ -762,3 +762,46 @@ def test_adamw_and_sum_squares_match_cpu(fhp, oracle, tb):
     actual = tb.GlobalSumSquares(ts)
     assert abs(actual - expected) / max(1.0, expected) < 2e-5
     assert tb.GlobalSumSquares([]) == 0.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(1, 1), (64, 63), (65, 64), (33, 65), (2049, 257), (700, 513), (2100, 769),
+                                       (5, 1024), (300, 1025)])
+def test_column_reductions_chunks_and_widths(fhp, tb, rows, cols):
+    """SumRows and LayerNormBackward (dx, dw, db) around their row chunks and row widths against
+    float64.  A float32 sum of n terms in any order is off by at most n 2^-24 times the sum of their
+    sizes; sums in several chains stay under a quarter of that.  dx has a few roundings per element."""
+    g = np.random.default_rng(rows * 31 + cols)
+    d, x = g.standard_normal((2, rows, cols)).astype(np.float32)
+    w = (1 + 0.1 * g.standard_normal(cols)).astype(np.float32)
+    prior = g.standard_normal((3, cols)).astype(np.float32)
+    x64, d64 = x.astype(np.float64), d.astype(np.float64)
+    mean = x64.mean(1).astype(np.float32)
+    rstd = (1 / np.sqrt(x64.var(1) + 1e-5)).astype(np.float32)
+    xh = (x64 - mean[:, None].astype(np.float64)) * rstd[:, None].astype(np.float64)
+    sums = [dup(fhp, v, cols) for v in prior]
+    dt, dx = dup(fhp, d, rows, cols), fhp.Tensor(rows, cols)
+    tb.SumRows(dt, sums[0], rows, cols)
+    tb.LayerNormBackward(dt, dup(fhp, x, rows, cols), dup(fhp, w, cols), dup(fhp, mean, rows), dup(fhp, rstd, rows), dx,
+                         sums[1], sums[2], rows, cols)
+    for t in sums + [dx]:
+        tb.EnsureHostCurrent(t)
+    for t, p, terms in zip(sums, prior.astype(np.float64), (d64, d64 * xh, d64)):
+        bound = 2.0 ** -24 * (4 + rows / 4) * (np.abs(terms).sum(0) + np.abs(p))
+        assert np.all(np.abs(t.Data - p - terms.sum(0)) <= bound)
+    dxh = d64 * w
+    want = rstd[:, None] * (dxh - dxh.mean(1, keepdims=True) - xh * (dxh * xh).mean(1, keepdims=True))
+    size = np.abs(rstd[:, None]) * (np.abs(dxh) + np.abs(dxh).mean(1, keepdims=True) +
+                                    np.abs(xh) * np.abs(dxh * xh).mean(1, keepdims=True))
+    assert np.all(np.abs(dx.Data.reshape(rows, cols) - want) <= 2.0 ** -24 * (8 + cols / 16) * size)
+
+
+@pytest.mark.gpu
+def test_global_sum_squares_over_many_tensors(fhp, tb):
+    """More tensors than one launch takes, an empty one among them, each end of the block counts: double sums."""
+    g = np.random.default_rng(9)
+    sizes = [1, 255, 8192, 8193, 0, 100003, 5000000] + [7 + i for i in range(130)]
+    data = [g.standard_normal(n).astype(np.float32) for n in sizes]
+    want = sum(float((v.astype(np.float64) ** 2).sum()) for v in data)
+    got = tb.GlobalSumSquares([dup(fhp, v, len(v)) for v in data])
+    assert abs(got - want) <= 1e-12 * want
