@@ -805,3 +805,95 @@ def test_global_sum_squares_over_many_tensors(fhp, tb):
     want = sum(float((v.astype(np.float64) ** 2).sum()) for v in data)
     got = tb.GlobalSumSquares([dup(fhp, v, len(v)) for v in data])
     assert abs(got - want) <= 1e-12 * want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 64), (7, 65), (130, 129), (9, 384), (6, 385), (4, 769), (5, 1024),
+                                       (3, 1025)])
+def test_row_kernels_widths(fhp, tb, rows, cols):
+    """Softmax forward (plain and causal) and backward and LayerNorm forward at the edges of the row
+    widths that pick a kernel, against float64.  expf, a sum over the row and a few products: 16 roundings
+    and cols / 64 in a lane's chain; the backward's difference is against the size of its two terms."""
+    g = np.random.default_rng(rows * 7 + cols)
+    x, d = g.standard_normal((2, rows, cols)).astype(np.float32)
+    ulp = 2.0 ** -24 * (16 + cols / 16)
+    for causal in (False, True):
+        z = x.astype(np.float64) * (0.3 if causal else 1.0)
+        if causal:
+            z = np.where(np.arange(cols)[None, :] <= (np.arange(rows) % cols)[:, None], z, -np.inf)
+        p = np.exp(z - z.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        t = dup(fhp, x, rows, cols)
+        if causal:
+            tb.ScaledCausalSoftmaxForward(t, rows, cols, 0.3)
+        else:
+            tb.SoftmaxForward(t, rows, cols)
+        tb.EnsureHostCurrent(t)
+        got = t.Data.reshape(rows, cols).astype(np.float64)
+        assert np.all(np.abs(got - p) <= (ulp + 2.0 ** -22 * np.abs(x)) * p)  # the scaled score's own rounding too
+        dx = fhp.Tensor(rows, cols)
+        tb.ScaledSoftmaxBackward(dup(fhp, d, rows, cols), t, dx, rows, cols, 0.3)
+        tb.EnsureHostCurrent(dx)
+        dot = (got * d).sum(1, keepdims=True)
+        size = 0.3 * got * (np.abs(d) + np.abs(got * d).sum(1, keepdims=True))
+        assert np.all(np.abs(dx.Data.reshape(rows, cols) - 0.3 * got * (d - dot)) <= ulp * size)
+    w, b = (1 + 0.1 * g.standard_normal((2, cols))).astype(np.float32)
+    out, mean, rstd = fhp.Tensor(rows, cols), fhp.Tensor(rows), fhp.Tensor(rows)
+    tb.LayerNormForward(dup(fhp, x, rows, cols), dup(fhp, w, cols), dup(fhp, b, cols), out, mean, rstd, rows, cols, 1e-5)
+    tb.EnsureHostCurrent(out)
+    x64 = x.astype(np.float64)
+    rs = 1 / np.sqrt(x64.var(1, keepdims=True) + 1e-5)
+    want = (x64 - x64.mean(1, keepdims=True)) * rs * w + b
+    size = (np.abs(x64) + np.abs(x64).mean(1, keepdims=True)) * rs * np.abs(w) + np.abs(b)
+    assert np.all(np.abs(out.Data.reshape(rows, cols) - want) <= ulp * size)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,V", [(3, 1), (2, 1023), (5, 4096), (3, 4097), (4, 16385), (2, 32768), (2, 32769)])
+def test_cross_entropy_vocabulary_widths(fhp, tb, T, V):
+    """CrossEntropy forward (in place) and backward at the edges of the vocabularies that pick a kernel."""
+    g = np.random.default_rng(T + V)
+    x = (3 * g.standard_normal((T, V))).astype(np.float32)
+    x[0, V // 2] = -np.inf if V > 1 else 0.0
+    tg = g.integers(0, V, T).astype(np.int32)
+    tg[-1] = -1  # ignored
+    if V > 1 and tg[0] == V // 2:
+        tg[0] = 0
+    t = dup(fhp, x, T, V)
+    loss = tb.CrossEntropyForward(t, tg, t, T, V, -1)
+    z = x.astype(np.float64)
+    p = np.exp(z - z.max(1, keepdims=True))
+    s = p.sum(1, keepdims=True)
+    p /= s
+    on = tg >= 0
+    nll = np.log(s[:, 0]) + z.max(1) - z[np.arange(T), np.maximum(tg, 0)]
+    assert abs(loss - nll[on].mean()) <= 2.0 ** -24 * 32 * np.abs(nll[on]).mean() + 1e-6
+    tb.EnsureHostCurrent(t)
+    got = t.Data.reshape(T, V).astype(np.float64)
+    assert np.all(np.abs(got - p) <= 2.0 ** -24 * (24 + V / 1024) * p + 2.0 ** -22 * p * np.abs(np.where(p > 0, z, 0)))
+    tb.CrossEntropyBackward(t, tg, t, T, V, -1)
+    tb.EnsureHostCurrent(t)
+    one = np.zeros((T, V))
+    one[np.arange(T)[on], tg[on]] = 1
+    want = np.where(on[:, None], got - one, 0) / on.sum()
+    assert np.all(np.abs(t.Data.reshape(T, V) - want) <= 2.0 ** -23 * (got + one) / on.sum())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,T,H,hd,pad", [(1, 1, 1, 1, 0), (2, 5, 3, 6, 2), (3, 17, 2, 64, 0), (1, 300, 4, 20, 1),
+                                              (2, 9, 5, 8, 4)])
+def test_head_packing_widths(fhp, tb, batch, T, H, hd, pad):
+    """Head packing in both directions, by 16-byte and by single loads (odd widths and offsets), exactly."""
+    d = H * hd
+    src = np.random.default_rng(T + hd).standard_normal((batch, T, d + 2 * pad)).astype(np.float32)
+    want = src[:, :, pad:pad + d].reshape(batch, T, H, hd).transpose(0, 2, 1, 3)
+    out = fhp.Tensor(batch * H * T, hd)
+    tb.PackHeads(dup(fhp, src, batch * T, d + 2 * pad), out, batch, T, H, hd, pad)
+    back = dup(fhp, 0 * src - 1, batch * T, d + 2 * pad)
+    tb.UnpackHeads(out, back, batch, T, H, hd, pad)
+    tb.EnsureHostCurrent(out)
+    tb.EnsureHostCurrent(back)
+    np.testing.assert_array_equal(out.Data.reshape(want.shape), want)
+    full = -np.ones_like(src)
+    full[:, :, pad:pad + d] = src[:, :, pad:pad + d]
+    np.testing.assert_array_equal(back.Data.reshape(src.shape), full)
