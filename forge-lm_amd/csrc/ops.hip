@@ -23,6 +23,7 @@
 #include <stdio.h>
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "common.hpp"
@@ -569,8 +570,53 @@ __global__ void k_embedding_forward(const float* __restrict__ table, const int* 
   for (int c = threadIdx.x; c < D; c += blockDim.x) out[(size_t)t * D + c] = src[c];
 }
 
-// dTable[id] += dOut[t] for the positions t of each distinct id, ascending:
-// uniq[u] is the id, pos[start[u] .. start[u+1]) its positions in order.
+// dTable[id] += dOut[t] for the positions t of each distinct id, in ascending order (the CPU
+// loop's sums).  Block t works if no earlier position has its id: it lists the later ones that
+// do in LDS, in order, and each thread adds up its columns with 8 loads in flight (a text's
+// commonest token comes up often: 80 of 2048 positions one load at a time took 15 us).  The ids
+// are compared n^2 times in all, 16 to a thread at n = 2048; up to kScatterIds positions that is
+// less than sorting them on the host took.
+constexpr int kScatterIds = 8192;
+__global__ __launch_bounds__(256) void k_embedding_scatter(const float* __restrict__ dout, const int* __restrict__ idx,
+                                                           int n, float* __restrict__ dtable, int D) {
+  __shared__ int list[kScatterIds];
+  __shared__ int counts[4];
+  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int id = idx[t];
+  int dup = 0;
+  for (int j = tid; j < t; j += 256) dup |= idx[j] == id;
+  if (__syncthreads_or(dup)) return;
+  int m = 0;  // listed so far
+  for (int j0 = t; j0 < n; j0 += 256) {
+    const bool hit = j0 + tid < n && idx[min(j0 + tid, n - 1)] == id;
+    const unsigned long long mask = __ballot(hit);
+    if (lane == 0) counts[w] = __popcll(mask);
+    __syncthreads();
+    int at = m + __popcll(mask & ((1ull << lane) - 1));
+    for (int i = 0; i < 4; i++) {
+      if (i < w) at += counts[i];
+      m += counts[i];
+    }
+    if (hit) list[at] = j0 + tid;
+    __syncthreads();
+  }
+  for (int c = tid; c < D; c += 256) {
+    float s = dtable[(size_t)id * D + c];
+    int k = 0;
+    for (; k + 8 <= m; k += 8) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[i] = dout[(size_t)list[k + i] * D + c];
+#pragma unroll
+      for (int i = 0; i < 8; i++) s = s + v[i];
+    }
+    for (; k < m; k++) s = s + dout[(size_t)list[k] * D + c];
+    dtable[(size_t)id * D + c] = s;
+  }
+}
+
+// The same for more positions, grouped on the host: uniq[u] is the id, pos[start[u] ..
+// start[u+1]) its positions in order.
 __global__ void k_embedding_backward(const float* __restrict__ dout, const int* __restrict__ uniq,
                                      const int* __restrict__ start, const int* __restrict__ pos,
                                      float* __restrict__ dtable, int D) {
@@ -762,11 +808,19 @@ __global__ void k_adamw(float* __restrict__ w, const float* __restrict__ g, floa
 
 }  // namespace
 
+constexpr int kStages = 8;
+constexpr size_t kStageBytes = (size_t)1 << 16;  // 16384 indices; larger arrays are copied with a wait
+
 // Per-context state of the op entry points: device scratch for uploaded index
 // arrays and reduction partials, and the loss accumulation.
 struct OpsState {
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
+  // pinned host memory that uploads leave from, so that a call returns without waiting for
+  // its copy: kStages areas in turn, each with an event that says its last copy is done
+  char* stage = nullptr;
+  hipEvent_t stage_done[kStages] = {};
+  int stage_next = 0;
   double* acc = nullptr;  // device loss accumulator + a result slot
   bool accumulating = false;
   long long accumulated_targets = 0;
@@ -776,6 +830,9 @@ void ops_state_free(OpsState* o) {
   if (!o) return;
   if (o->scratch) (void)hipFree(o->scratch);
   if (o->acc) (void)hipFree(o->acc);
+  for (hipEvent_t e : o->stage_done)
+    if (e) (void)hipEventDestroy(e);
+  if (o->stage) (void)hipHostFree(o->stage);
   delete o;
 }
 
@@ -855,14 +912,41 @@ int op_launched(const char* what) {
 #define OPS_ARG(cond, ...) \
   if (!(cond)) return set_err(FH_ERR_INVALID, __VA_ARGS__)
 
+// Host ints to dev on the context's stream; the host array may go away on return.  It is
+// copied into the next staging area (16 KB of targets or ids in a microsecond), whose event
+// bounds how far the host runs ahead: waiting for each copy cost a training step 20-30 us per
+// upload with the device idle.
+int copy_ints(fh_context* c, OpsState* o, const int32_t* host, size_t n, int* dev) {
+  hipStream_t st = context_stream(c);
+  const size_t bytes = n * sizeof(int32_t);
+  if (bytes > kStageBytes) {
+    HIP_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    return FH_OK;
+  }
+  if (!o->stage) {
+    void* p = nullptr;
+    HIP_TRY(hipHostMalloc(&p, kStages * kStageBytes, hipHostMallocDefault));
+    o->stage = static_cast<char*>(p);
+  }
+  const int k = o->stage_next;
+  if (o->stage_done[k])
+    HIP_TRY(hipEventSynchronize(o->stage_done[k]));
+  else
+    HIP_TRY(hipEventCreateWithFlags(&o->stage_done[k], hipEventDisableTiming));
+  char* from = o->stage + k * kStageBytes;
+  std::memcpy(from, host, bytes);
+  HIP_TRY(hipMemcpyAsync(dev, from, bytes, hipMemcpyHostToDevice, st));
+  HIP_TRY(hipEventRecord(o->stage_done[k], st));
+  o->stage_next = (k + 1) % kStages;
+  return FH_OK;
+}
+
 int upload_ints(fh_context* c, OpsState* o, const int32_t* host, size_t n, int** dev) {
   void* p = nullptr;
   FH_TRY(ops_scratch(c, o, n * sizeof(int32_t), &p));
-  // synchronous: the caller's array may go away as soon as the entry point returns
-  HIP_TRY(hipMemcpyAsync(p, host, n * sizeof(int32_t), hipMemcpyHostToDevice, context_stream(c)));
-  HIP_TRY(hipStreamSynchronize(context_stream(c)));
   *dev = static_cast<int*>(p);
-  return FH_OK;
+  return copy_ints(c, o, host, n, *dev);
 }
 
 // the partial sums of a split K take at most this much of the context's scratch (64 MB)
@@ -1133,6 +1217,13 @@ int fh_op_embedding_backward(fh_context* c, const void* dout, const int32_t* ind
     if (indices[t] < 0 || indices[t] >= table_rows)
       return set_err(FH_ERR_RANGE, "index %d at position %d outside the table's %d rows", indices[t], t, table_rows);
   if (n == 0) return FH_OK;
+  if (n <= kScatterIds) {
+    int* di = nullptr;
+    FH_TRY(upload_ints(c, ops_, indices, (size_t)n, &di));
+    hipLaunchKernelGGL(k_embedding_scatter, dim3(n), dim3(256), 0, st_, static_cast<const float*>(dout), di, n,
+                       static_cast<float*>(dtable), D);
+    return op_launched("embedding backward");
+  }
   // group the positions by id, ascending within each id
   std::vector<int> order(n);
   for (int t = 0; t < n; t++) order[t] = t;
@@ -1179,8 +1270,7 @@ int fh_op_cross_entropy_forward(fh_context* c, const void* logits, const int32_t
   FH_TRY(ops_scratch(c, ops_, (size_t)T * (sizeof(int32_t) + sizeof(float)), &p));
   int* dt = static_cast<int*>(p);
   float* nll = reinterpret_cast<float*>(dt + T);
-  HIP_TRY(hipMemcpyAsync(dt, targets, (size_t)T * sizeof(int32_t), hipMemcpyHostToDevice, st_));
-  HIP_TRY(hipStreamSynchronize(st_));
+  FH_TRY(copy_ints(c, ops_, targets, (size_t)T, dt));
   const float* lg = static_cast<const float*>(logits);
   float* pr = static_cast<float*>(probs);
   if (V <= 1024 * 4)

@@ -201,7 +201,10 @@ class HipTensorBackend:
     def UnpackQkvHeads(self, q, k, v, dst, batch, T, nHeads, headDim):
         """ITensorBackend.cs:68-76."""
         d = nHeads * headDim
-        self.Zero(dst)
+        if dst.Cols == 3 * d and dst.Length == batch * T * 3 * d:
+            self._write(dst)  # the three slices fill it: no zeros to write, no host copy to upload
+        else:
+            self.Zero(dst)
         self.UnpackHeads(q, dst, batch, T, nHeads, headDim, 0)
         self.UnpackHeads(k, dst, batch, T, nHeads, headDim, d)
         self.UnpackHeads(v, dst, batch, T, nHeads, headDim, 2 * d)

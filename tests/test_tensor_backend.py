@@ -897,3 +897,58 @@ def test_head_packing_widths(fhp, tb, batch, T, H, hd, pad):
     full = -np.ones_like(src)
     full[:, :, pad:pad + d] = src[:, :, pad:pad + d]
     np.testing.assert_array_equal(back.Data.reshape(src.shape), full)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,D,vocab", [(1, 3, 5), (255, 64, 7), (257, 300, 2), (2048, 40, 1000), (8192, 8, 50),
+                                       (8193, 8, 50)])
+def test_embedding_backward_repeated_ids(fhp, tb, n, D, vocab):
+    """Every position of a repeated id, in ascending order: the sums of a sequential float32 loop, exactly,
+    grouped on the device and (past 8192 positions) on the host."""
+    g = np.random.default_rng(n)
+    ids = (g.random(n) ** 3 * vocab).astype(np.int32)
+    dout = g.standard_normal((n, D)).astype(np.float32)
+    want = g.standard_normal((vocab, D)).astype(np.float32)
+    t = dup(fhp, want, vocab, D)
+    for i, r in zip(ids, dout):
+        want[i] += r
+    tb.EmbeddingBackward(dup(fhp, dout, n, D), ids, t, D)
+    tb.EnsureHostCurrent(t)
+    np.testing.assert_array_equal(t.Data.reshape(vocab, D), want)
+
+
+@pytest.mark.gpu
+def test_index_uploads_run_ahead(fhp, tb):
+    """More uploads than there are staging areas before anything waits, of changing sizes, from one host
+    array that is overwritten after each call."""
+    g = np.random.default_rng(3)
+    table = g.standard_normal((100, 4)).astype(np.float32)
+    t = dup(fhp, table, 100, 4)
+    buf = np.empty(20000, np.int32)
+    outs, want = [], []
+    for i in range(40):
+        n = (1 + 37 * i) if i % 7 else 20000
+        ids = buf[:n]
+        ids[:] = g.integers(0, 100, n)
+        outs.append(fhp.Tensor(n, 4))
+        want.append(table[ids])
+        tb.EmbeddingForward(t, ids, outs[-1], 4)
+    for o, w in zip(outs, want):
+        tb.EnsureHostCurrent(o)
+        np.testing.assert_array_equal(o.Data.reshape(w.shape), w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(6, 12), (8, 12), (6, 15)])
+def test_unpack_qkv_zeroes_what_it_does_not_fill(fhp, tb, rows, cols):
+    """dst of exactly the three slices, with rows past them, and with wider rows: zeros around the slices."""
+    g = np.random.default_rng(cols)
+    B, T, H, hd = 2, 3, 2, 2
+    qkv = [dup(fhp, g.standard_normal((B * H * T, hd)), B * H * T, hd) for _ in range(3)]
+    dst = dup(fhp, np.full((rows, cols), 5.0), rows, cols)
+    tb.UnpackQkvHeads(*qkv, dst, B, T, H, hd)
+    tb.EnsureHostCurrent(dst)
+    want = np.zeros((rows, cols), np.float32)
+    for i, t in enumerate(qkv):
+        want[:B * T, 4 * i:4 * i + 4] = t.Data.reshape(B, H, T, hd).transpose(0, 2, 1, 3).reshape(B * T, 4)
+    np.testing.assert_array_equal(dst.Data.reshape(rows, cols), want)
