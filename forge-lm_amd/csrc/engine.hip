@@ -241,6 +241,7 @@ struct fh_session {
   // activations (rows = B*ctx)
   float *x = nullptr, *x2 = nullptr, *xn = nullptr, *qkv = nullptr, *o = nullptr, *h = nullptr;
   float *part = nullptr, *apart = nullptr, *logits = nullptr, *work = nullptr;
+  size_t short_floats = 0;
   size_t part_floats = 0;
   // bf16 sessions: arrival counters of the window mlp.proj with K split in two
   // (one per 256 x 256 tile, zero between launches; o holds the first halves' sums)
@@ -342,6 +343,19 @@ int check_launch(hipError_t e, const char* what) {
 
 #define LAUNCH(expr) FH_TRY(check_launch((expr), #expr))
 
+// fp32 products of more than kSplitRows rows run on the split GEMM, fewer on the fp32 MFMA
+// GEMM, whose 32-row tile pads less (a 98M window of 20 rows 0.69 against 0.77 ms; of 66
+// rows 0.93 against 1.05, of 333 1.69 against 1.89, of 1024 3.04 against 3.91)
+constexpr int kSplitRows = 32;
+// room for the partial sums of a split K in fp32 sessions, 32 MB (8 MB: 1024 rows 3.19 ms,
+// 3 x 700 rows 4.10 against 3.84; 64 MB no faster)
+constexpr size_t kPartFloats = (size_t)8 << 20;
+
+template <typename WT>
+bool use_split(int M) {
+  return std::is_same<WT, float>::value && M > kSplitRows;
+}
+
 // y = epi(x @ W + b) (+ res) for registry matrix `slot`: split-K GEMV for up to
 // 4 rows, the MFMA GEMM on the transposed copy above that.
 template <typename WT>
@@ -353,6 +367,9 @@ int linear(fh_session* s, const float* x, int M, int K, size_t slot, int N, cons
     int splits = std::max(1, std::min(64, K / 16));
     LAUNCH(launch_gemv_splitk<WT>(st, x, M, K, s->w<WT>(slot), N, s->part, splits, &S));
     LAUNCH(launch_splitk_epilogue(st, s->part, S, M, N, b, epi, res, y));
+  } else if (use_split<WT>(M)) {
+    LAUNCH(launch_gemm_split(st, 1, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), 1, M, K, N, b,
+                             epi == EPI_GELU, res, y, s->part, s->part_floats, s->ctx->props.multiProcessorCount));
   } else if (K % 32 == 0) {
     LAUNCH(launch_gemm_mfma<WT>(st, x, M, K, s->wt<WT>(slot), N, b, epi, res, y, s->part, s->part_floats,
                                 s->ctx->props.multiProcessorCount));
@@ -370,6 +387,9 @@ int linear_parts(fh_session* s, const float* x, int M, int K, size_t slot, int N
   if (M <= 4) {
     const int splits = std::max(1, std::min(64, K / 16));
     LAUNCH(launch_gemv_splitk<WT>(st, x, M, K, s->w<WT>(slot), N, s->part, splits, S));
+  } else if (use_split<WT>(M)) {
+    LAUNCH(launch_gemm_split_parts(st, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), M, K, N, s->part,
+                                   s->part_floats, s->ctx->props.multiProcessorCount, S));
   } else {
     LAUNCH(launch_gemm_mfma_split<WT>(st, x, M, K, s->wt<WT>(slot), N, s->part, s->part_floats,
                                       s->ctx->props.multiProcessorCount, S));
@@ -506,7 +526,7 @@ int enqueue_layers_window(fh_session* s, int T, RowSrc src, LastRows* last) {
     if (s->bf16_act && M >= 256 && D % 64 == 0 && D == 64 * H)
       return enqueue_layers_window_bf16(s, T, src, last);
   }
-  if (M > 4 && D % 32 == 0 && D <= 1024 && (size_t)M * 3 * D <= s->part_floats) {
+  if (M > 4 && D % 32 == 0 && D <= 1024 && (size_t)M * 3 * D <= s->short_floats) {
     // short windows: the split-K reductions also store K/V and apply LN2 and the
     // next layer's LN1, as in batched decode (the last mlp.proj keeps its residual
     // epilogue: LN_f runs on the last rows only)
@@ -1183,8 +1203,10 @@ int fh_session_create(fh_context* c, const fh_model_desc* desc, fh_session** out
   // split-K partials: the GEMV path (up to 64 splits of 4 rows), the MFMA GEMM's
   // small-M split (up to 8 splits of 64 rows of the widest layer), and at least
   // one unsplit product of every decode row (the batched decode's split GEMMs need
-  // B x 3D; the split count shrinks to what fits)
-  sp->part_floats = std::max({(size_t)64 * 4 * 4 * D, (size_t)8 * 64 * 4 * D, (size_t)B * 4 * D});
+  // B x 3D; the split count shrinks to what fits).  short_floats also bounds the windows
+  // whose reductions carry the kernels after them; fp32 sessions have more room for splits
+  sp->short_floats = std::max({(size_t)64 * 4 * 4 * D, (size_t)8 * 64 * 4 * D, (size_t)B * 4 * D});
+  sp->part_floats = std::max(sp->short_floats, desc->dtype == FH_DTYPE_F32 ? kPartFloats : 0);
   if ((rc = dev_alloc(&sp->x, rows * D)) || (rc = dev_alloc(&sp->x2, rows * D)) || (rc = dev_alloc(&sp->xn, rows * D)) ||
       (rc = dev_alloc(&sp->qkv, rows * 3 * D)) || (rc = dev_alloc(&sp->o, rows * D)) ||
       (rc = dev_alloc(&sp->h, rows * 4 * D)) || (rc = dev_alloc(&sp->part, sp->part_floats)) ||
