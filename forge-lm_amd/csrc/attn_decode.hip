@@ -213,4 +213,119 @@ template hipError_t launch_attn_decode_wide<float>(hipStream_t, RowSrc, const fl
 template hipError_t launch_attn_decode_wide<bf16_t>(hipStream_t, RowSrc, const float*, int, int, int, int,
                                                     const bf16_t*, const bf16_t*, float*, float*, bool, const QkvParts*);
 
+namespace {
+
+// Decode attention of one (sequence, head) per block, for caches of at most 256 positions:
+// L lanes share a key (16 bytes of its row each), a wave takes 64 / L keys at a time and its
+// four waves every fourth group, so all K and V rows a block can need are in flight at
+// once, with the step counter that says how many count.  Latency-bound: one launch of 4 us
+// where 64-key chunks and their combination took 9 + 4 (4 heads of 32, ctx 128).
+template <typename KT, int L>
+__global__ __launch_bounds__(256) void k_attn_decode_one(RowSrc src, const float* __restrict__ qkv, int d, int H,
+                                                         int ctx, const KT* __restrict__ kc,
+                                                         const KT* __restrict__ vc, float* __restrict__ o) {
+  constexpr int VEC = 16 / sizeof(KT), G = 64 / L, NIT = L;  // 4 G NIT = 256 keys
+  __shared__ float red[4], sums[4];
+  __shared__ float part[4][L * VEC];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x, b = blockIdx.y, hd = d / H;
+  const int e0 = lane % L * VEC, grp = lane / L;
+  const size_t head = ((size_t)b * H + h) * ctx * hd;
+  const int range = ctx * hd * (int)sizeof(KT);
+  const __amdgpu_buffer_rsrc_t rk =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<KT*>(kc + head), (short)0, range, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<KT*>(vc + head), (short)0, range, 0x00020000);
+  u32x4_t kr[NIT], vr[NIT];
+#pragma unroll
+  for (int i = 0; i < NIT; i++) {
+    const int key = (i * 4 + w) * G + grp;
+    const int off = e0 < hd ? (key * hd + e0) * (int)sizeof(KT) : range;  // at or past range: 0
+    kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0);
+    vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, off, 0, 0);
+  }
+  const int nkeys = min(ctx, src.pos_off + src.pos_mul * *src.step + 1);
+  const float* qp = qkv + (size_t)b * 3 * d + h * hd;
+  float q[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; j++) q[j] = e0 + j < hd ? qp[e0 + j] : 0.f;
+  auto elem = [](const u32x4_t& v, int j) {
+    if constexpr (sizeof(KT) == 4)
+      return __uint_as_float(v[j]);
+    else
+      return __uint_as_float(j & 1 ? v[j / 2] & 0xffff0000u : v[j / 2] << 16);
+  };
+  const float scale = 1.f / sqrtf((float)hd);
+  float s[NIT], m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < NIT; i++) {
+    float dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < VEC; j++) dot = fmaf(q[j], elem(kr[i], j), dot);
+#pragma unroll
+    for (int x = L / 2; x > 0; x >>= 1) dot += __shfl_xor(dot, x, 64);
+    s[i] = (i * 4 + w) * G + grp < nkeys ? dot * scale : -INFINITY;  // rows past nkeys hold anything
+    m = fmaxf(m, s[i]);
+  }
+  m = wave_max_dpp(m);
+  if (lane == 0) red[w] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float l = 0.f, acc[VEC];
+#pragma unroll
+  for (int j = 0; j < VEC; j++) acc[j] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NIT; i++) {
+    const bool on = (i * 4 + w) * G + grp < nkeys;
+    const float p = on ? expf(s[i] - m) : 0.f;
+    l += p;
+#pragma unroll
+    for (int j = 0; j < VEC; j++) acc[j] = on ? fmaf(p, elem(vr[i], j), acc[j]) : acc[j];
+  }
+  l = wave_sum_dpp(lane % L == 0 ? l : 0.f);
+  if (lane == 0) sums[w] = l;
+#pragma unroll
+  for (int j = 0; j < VEC; j++) {
+#pragma unroll
+    for (int x = L; x < 64; x <<= 1) acc[j] += __shfl_xor(acc[j], x, 64);
+    if (lane < L) part[w][e0 + j] = acc[j];
+  }
+  __syncthreads();
+  const int e = threadIdx.x;
+  if (e < hd)
+    o[(size_t)b * d + h * hd + e] =
+        (part[0][e] + part[1][e] + part[2][e] + part[3][e]) / (sums[0] + sums[1] + sums[2] + sums[3]);
+}
+
+}  // namespace
+
+bool attn_decode_one_fits(int d, int H, int ctx, int esize) {
+  const int vec = 16 / esize, hd = d / H;
+  return ctx <= 256 && hd % vec == 0 && hd <= 16 * vec;
+}
+
+template <typename KT>
+hipError_t launch_attn_decode_one(hipStream_t st, RowSrc src, const float* qkv, int B, int d, int H, int ctx,
+                                  const KT* kc, const KT* vc, float* o) {
+  if (B <= 0 || H <= 0 || d <= 0 || d % H != 0 || ctx <= 0 || !attn_decode_one_fits(d, H, ctx, sizeof(KT)) || !qkv ||
+      !kc || !vc || !o || !src.step)
+    return hipErrorInvalidValue;
+  const int pieces = d / H / (16 / (int)sizeof(KT));
+  const dim3 grid(H, B);
+  if (pieces <= 2)
+    hipLaunchKernelGGL((k_attn_decode_one<KT, 2>), grid, dim3(256), 0, st, src, qkv, d, H, ctx, kc, vc, o);
+  else if (pieces <= 4)
+    hipLaunchKernelGGL((k_attn_decode_one<KT, 4>), grid, dim3(256), 0, st, src, qkv, d, H, ctx, kc, vc, o);
+  else if (pieces <= 8)
+    hipLaunchKernelGGL((k_attn_decode_one<KT, 8>), grid, dim3(256), 0, st, src, qkv, d, H, ctx, kc, vc, o);
+  else
+    hipLaunchKernelGGL((k_attn_decode_one<KT, 16>), grid, dim3(256), 0, st, src, qkv, d, H, ctx, kc, vc, o);
+  return hipGetLastError();
+}
+
+template hipError_t launch_attn_decode_one<float>(hipStream_t, RowSrc, const float*, int, int, int, int, const float*,
+                                                  const float*, float*);
+template hipError_t launch_attn_decode_one<bf16_t>(hipStream_t, RowSrc, const float*, int, int, int, int,
+                                                   const bf16_t*, const bf16_t*, float*);
+
 }  // namespace fh

@@ -356,17 +356,13 @@ bool use_split(int M) {
   return std::is_same<WT, float>::value && M > kSplitRows;
 }
 
-// y = epi(x @ W + b) (+ res) for registry matrix `slot`: split-K GEMV for up to
-// 4 rows, the MFMA GEMM on the transposed copy above that.
+// y = epi(x @ W + b) (+ res) for registry matrix `slot`: the GEMV for up to 4 rows, the MFMA GEMM on the transposed copy above that.
 template <typename WT>
 int linear(fh_session* s, const float* x, int M, int K, size_t slot, int N, const float* b, int epi, const float* res,
            float* y) {
   hipStream_t st = s->ctx->stream;
   if (M <= 4) {
-    int S = 0;
-    int splits = std::max(1, std::min(64, K / 16));
-    LAUNCH(launch_gemv_splitk<WT>(st, x, M, K, s->w<WT>(slot), N, s->part, splits, &S));
-    LAUNCH(launch_splitk_epilogue(st, s->part, S, M, N, b, epi, res, y));
+    LAUNCH(launch_gemv<WT>(st, x, M, K, s->wt<WT>(slot), N, nullptr, nullptr, 0.f, b, epi, res, y));
   } else if (use_split<WT>(M)) {
     LAUNCH(launch_gemm_split(st, 1, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), 1, M, K, N, b,
                              epi == EPI_GELU, res, y, s->part, s->part_floats, s->ctx->props.multiProcessorCount));
@@ -379,15 +375,21 @@ int linear(fh_session* s, const float* x, int M, int K, size_t slot, int N, cons
   return FH_OK;
 }
 
-// x @ W for registry matrix `slot` into split-K partials s->part (no bias or
+// y = epi(LN(x) @ W + b) for up to 4 rows: the LayerNorm of registry slots ln, ln + 1 in the GEMV
+template <typename WT>
+int linear_ln(fh_session* s, const float* x, int M, size_t ln, size_t slot, int N, const float* b, int epi, float* y,
+              const QkvStore<WT>* kv = nullptr) {
+  LAUNCH(launch_gemv<WT>(s->ctx->stream, x, M, s->d.d_model, s->wt<WT>(slot), N, s->v(ln), s->v(ln + 1), 1e-5f, b, epi,
+                         nullptr, y, kv));
+  return FH_OK;
+}
+
+// x @ W for registry matrix `slot` (more than 4 rows) into split-K partials s->part (no bias or
 // epilogue); *S receives the split count for the fused epilogue that sums them.
 template <typename WT>
 int linear_parts(fh_session* s, const float* x, int M, int K, size_t slot, int N, int* S) {
   hipStream_t st = s->ctx->stream;
-  if (M <= 4) {
-    const int splits = std::max(1, std::min(64, K / 16));
-    LAUNCH(launch_gemv_splitk<WT>(st, x, M, K, s->w<WT>(slot), N, s->part, splits, S));
-  } else if (use_split<WT>(M)) {
+  if (use_split<WT>(M)) {
     LAUNCH(launch_gemm_split_parts(st, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), M, K, N, s->part,
                                    s->part_floats, s->ctx->props.multiProcessorCount, S));
   } else {
@@ -401,21 +403,40 @@ int linear_parts(fh_session* s, const float* x, int M, int K, size_t slot, int N
 // (qkv + KV store, proj + LN2, mproj + the next LayerNorm, LN_f included).
 bool decode_fused_epilogues(const fh_session* s) {
   const int D = s->d.d_model;
-  return D <= 1024 && (s->B() <= 4 || D % 32 == 0);
+  return D <= 1024 && s->B() > 4 && D % 32 == 0;
 }
 
-// Tied head for B rows: logits = xn @ tok_emb^T.  tok_emb [V][d] is already
-// the transposed operand the MFMA GEMM reads, so more than 4 rows go there.
+// Tied head for B rows: logits = xn @ tok_emb^T.  tok_emb [V][d] is already the transposed
+// operand the GEMMs read: up to 4 rows take the GEMV (with x, LN_f of x instead of xn, in its
+// registers), more the MFMA GEMM.
 template <typename WT>
-int head(fh_session* s, int B) {
+int head(fh_session* s, int B, const float* x = nullptr) {
   hipStream_t st = s->ctx->stream;
   const int D = s->d.d_model, V = s->d.vocab_size;
-  if (B > 4 && D % 32 == 0) {
+  const size_t lf = s->idx_lnf();
+  if (B <= 4) {
+    LAUNCH(launch_gemv<WT>(st, x ? x : s->xn, B, D, s->w<WT>(s->idx_tok()), V, x ? s->v(lf) : nullptr,
+                           x ? s->v(lf + 1) : nullptr, 1e-5f, nullptr, EPI_NONE, nullptr, s->logits));
+  } else if (D % 32 == 0) {
     LAUNCH(launch_gemm_mfma<WT>(st, s->xn, B, D, s->w<WT>(s->idx_tok()), V, nullptr, EPI_NONE, nullptr, s->logits,
                                 s->part, s->part_floats, s->ctx->props.multiProcessorCount));
   } else {
     LAUNCH(launch_head<WT>(st, s->xn, B, D, s->w<WT>(s->idx_tok()), V, s->logits));
   }
+  return FH_OK;
+}
+
+// Attention of one row per sequence over the keys up to its position.
+template <typename WT>
+int decode_attention(fh_session* s, RowSrc src, const float* qkv, const WT* kc, const WT* vc) {
+  hipStream_t st = s->ctx->stream;
+  const int B = s->B(), D = s->d.d_model, H = s->d.n_heads, C = s->d.context_length;
+  if (attn_decode_one_fits(D, H, C, sizeof(WT)))
+    LAUNCH(launch_attn_decode_one<WT>(st, src, qkv, B, D, H, C, kc, vc, s->o));
+  else if (D == 64 * H)
+    LAUNCH(launch_attn_decode_wide<WT>(st, src, qkv, B, D, H, C, kc, vc, s->apart, s->o));
+  else
+    LAUNCH(launch_attn_decode<WT>(st, src, qkv, B, D, H, C, kc, vc, s->apart, 64, s->o));
   return FH_OK;
 }
 
@@ -443,7 +464,7 @@ bool last_rows_tail(const fh_session* s, int T) { return s->last_tail && T >= 3;
 template <typename WT, typename QT>
 int enqueue_last_rows(fh_session* s, int T, RowSrc src, int l, const QT* q, int q_ld, LastRows* last) {
   hipStream_t st = s->ctx->stream;
-  const int B = s->B(), D = s->d.d_model, H = s->d.n_heads, C = s->d.context_length;
+  const int B = s->B(), D = s->d.d_model;
   const size_t BD = (size_t)B * D;
   WT* kc = reinterpret_cast<WT*>(s->kc) + (size_t)l * s->kv_layer;
   WT* vc = reinterpret_cast<WT*>(s->vc) + (size_t)l * s->kv_layer;
@@ -455,10 +476,14 @@ int enqueue_last_rows(fh_session* s, int T, RowSrc src, int l, const QT* q, int 
   LAUNCH(launch_gather_rows<QT>(st, q, q_ld, T - 1, T, B, D, q1, 3 * D));
   LAUNCH(launch_gather_rows<float>(st, s->x, D, T - 1, T, B, D, x1, D));
   const RowSrc qsrc{src.tokens, src.step, src.tok_stride, src.tok_off + T - 1, T - 1, 0};
-  if (D == 64 * H)
-    LAUNCH(launch_attn_decode_wide<WT>(st, qsrc, q1, B, D, H, C, kc, vc, s->apart, s->o));
-  else
-    LAUNCH(launch_attn_decode<WT>(st, qsrc, q1, B, D, H, C, kc, vc, s->apart, 64, s->o));
+  FH_TRY(decode_attention<WT>(s, qsrc, q1, kc, vc));
+  if (B <= 4) {
+    FH_TRY(linear<WT>(s, s->o, B, D, s->idx_blk(l, 4), D, s->v(s->idx_blk(l, 5)), EPI_NONE, x1, x21));
+    FH_TRY(linear_ln<WT>(s, x21, B, s->idx_blk(l, 6), s->idx_blk(l, 8), 4 * D, s->v(s->idx_blk(l, 9)), EPI_GELU, f1));
+    FH_TRY(linear<WT>(s, f1, B, 4 * D, s->idx_blk(l, 10), D, s->v(s->idx_blk(l, 11)), EPI_NONE, x21, y1));
+    *last = LastRows{y1, 1, 0};
+    return FH_OK;
+  }
   if (decode_fused_epilogues(s)) {
     // as in batched decode: the split-K sums of attn.proj and mlp.proj fused with
     // the LayerNorm after them (LN2, LN_f), so xn holds the head's input on return
@@ -587,6 +612,23 @@ template <typename WT>
 int enqueue_layers_decode(fh_session* s, RowSrc src) {
   hipStream_t st = s->ctx->stream;
   const int B = s->B(), D = s->d.d_model, H = s->d.n_heads, C = s->d.context_length;
+  if (B <= 4) {
+    // five launches a layer: the LayerNorms run in the GEMVs that read them, the qkv GEMV
+    // stores the K/V row; x holds the input of LN_f on return
+    s->route |= FH_ROUTE_FUSED_EPILOGUES;
+    for (int l = 0; l < s->d.n_layers; l++) {
+      const QkvStore<WT> kv{src, 1, H, C, reinterpret_cast<WT*>(s->kc) + (size_t)l * s->kv_layer,
+                            reinterpret_cast<WT*>(s->vc) + (size_t)l * s->kv_layer};
+      FH_TRY(linear_ln<WT>(s, s->x, B, s->idx_blk(l, 0), s->idx_blk(l, 2), 3 * D, s->v(s->idx_blk(l, 3)), EPI_QKV,
+                           s->qkv, &kv));
+      FH_TRY(decode_attention<WT>(s, src, s->qkv, kv.kc, kv.vc));
+      FH_TRY(linear<WT>(s, s->o, B, D, s->idx_blk(l, 4), D, s->v(s->idx_blk(l, 5)), EPI_NONE, s->x, s->x2));
+      FH_TRY(linear_ln<WT>(s, s->x2, B, s->idx_blk(l, 6), s->idx_blk(l, 8), 4 * D, s->v(s->idx_blk(l, 9)), EPI_GELU,
+                           s->h));
+      FH_TRY(linear<WT>(s, s->h, B, 4 * D, s->idx_blk(l, 10), D, s->v(s->idx_blk(l, 11)), EPI_NONE, s->x2, s->x));
+    }
+    return FH_OK;
+  }
   if (decode_fused_epilogues(s)) {
     // each split-K reduction also does the work of the kernel after it; the last
     // mproj reduction applies LN_f, so xn holds the head's input on return
@@ -649,10 +691,7 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
       int S = 0;
       FH_TRY(linear_parts<WT>(s, s->xn, B, D, s->idx_blk(l, 2), 3 * D, &S));
       LAUNCH(launch_epilogue_qkv<WT>(st, s->part, S, B, D, s->v(s->idx_blk(l, 3)), s->qkv, src, 1, H, C, kc, vc));
-      if (D == 64 * H)
-        LAUNCH(launch_attn_decode_wide<WT>(st, src, s->qkv, B, D, H, C, kc, vc, s->apart, s->o));
-      else
-        LAUNCH(launch_attn_decode<WT>(st, src, s->qkv, B, D, H, C, kc, vc, s->apart, 64, s->o));
+      FH_TRY(decode_attention<WT>(s, src, s->qkv, kc, vc));
       FH_TRY(linear_parts<WT>(s, s->o, B, D, s->idx_blk(l, 4), D, &S));
       LAUNCH(launch_epilogue_ln(st, s->part, S, B, D, s->v(s->idx_blk(l, 5)), s->x, s->x2, s->v(s->idx_blk(l, 6)),
                                 s->v(s->idx_blk(l, 7)), s->xn, 1e-5f));
@@ -673,10 +712,7 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
     FH_TRY(linear<WT>(s, s->xn, B, D, s->idx_blk(l, 2), 3 * D, s->v(s->idx_blk(l, 3)), EPI_NONE, nullptr,
                       s->qkv));
     LAUNCH(launch_kv_store<WT>(st, src, s->qkv, B, 1, D, H, C, kc, vc));
-    if (D == 64 * H)
-      LAUNCH(launch_attn_decode_wide<WT>(st, src, s->qkv, B, D, H, C, kc, vc, s->apart, s->o));
-    else
-      LAUNCH(launch_attn_decode<WT>(st, src, s->qkv, B, D, H, C, kc, vc, s->apart, 64, s->o));
+    FH_TRY(decode_attention<WT>(s, src, s->qkv, kc, vc));
     FH_TRY(linear<WT>(s, s->o, B, D, s->idx_blk(l, 4), D, s->v(s->idx_blk(l, 5)), EPI_NONE, s->x, s->x2));
     LAUNCH(launch_layernorm(st, s->x2, B, B, 0, 0, s->v(s->idx_blk(l, 6)), s->v(s->idx_blk(l, 7)), s->xn, D, 1e-5f));
     FH_TRY(linear<WT>(s, s->xn, B, D, s->idx_blk(l, 8), 4 * D, s->v(s->idx_blk(l, 9)), EPI_GELU, nullptr,
@@ -725,9 +761,10 @@ int enqueue_window_step(fh_session* s, int T, const StepPlan& p) {
   LastRows last{};
   FH_TRY(enqueue_layers_window<WT>(s, T, src, &last));
   const size_t lf = s->idx_lnf();
-  if (last.x)
+  const bool ln_in_head = B <= 4 && last.x && last.r0 == 0 && last.stride == 1;
+  if (last.x && !ln_in_head)
     LAUNCH(launch_layernorm(st, last.x, B, 1, last.stride, last.r0, s->v(lf), s->v(lf + 1), s->xn, D, 1e-5f));
-  FH_TRY(head<WT>(s, B));
+  FH_TRY(head<WT>(s, B, ln_in_head ? last.x : nullptr));
   if (p.with_sample) LAUNCH(launch_sample(st, make_sample_args(s, p)));
   return FH_OK;
 }
@@ -786,9 +823,9 @@ int enqueue_decode_step(fh_session* s, const StepPlan& p) {
                             s->d.context_length, s->x));
     FH_TRY(enqueue_layers_decode<WT>(s, src));
     const size_t lf = s->idx_lnf();
-    if (!decode_fused_epilogues(s))
+    if (B > 4 && !decode_fused_epilogues(s))
       LAUNCH(launch_layernorm(st, s->x, B, 1, 1, 0, s->v(lf), s->v(lf + 1), s->xn, D, 1e-5f));
-    FH_TRY(head<WT>(s, B));
+    FH_TRY(head<WT>(s, B, s->x));
   }
   LAUNCH(launch_sample(st, make_sample_args(s, p)));
   return FH_OK;

@@ -243,54 +243,6 @@ __global__ __launch_bounds__(256) void k_epilogue_qkv(const float* __restrict__ 
     vc[dst] = from_f32<KT>(a);
 }
 
-// ---------------------------------------------------------------------------
-// split-K GEMV (M <= 4): each block owns a 64*VEC column tile and one K chunk;
-// each of its 4 waves walks every 4th row of the chunk with 16-byte loads.
-// ---------------------------------------------------------------------------
-template <typename WT, int MR>
-__global__ __launch_bounds__(256) void k_gemv_splitk(const float* __restrict__ x, int M, int K,
-                                                     const WT* __restrict__ W, int N, int kchunk,
-                                                     float* __restrict__ part) {
-  constexpr int VEC = 16 / sizeof(WT);
-  constexpr int TILE = 64 * VEC;
-  __shared__ float red[4][MR][TILE];
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int c0 = blockIdx.x * TILE + lane * VEC;
-  const int s = blockIdx.y;
-  const int k0 = s * kchunk, k1 = min(K, k0 + kchunk);
-  float acc[MR][VEC];
-#pragma unroll
-  for (int m = 0; m < MR; m++)
-#pragma unroll
-    for (int j = 0; j < VEC; j++) acc[m][j] = 0.f;
-  if (c0 < N) {
-#pragma unroll 4
-    for (int k = k0 + wv; k < k1; k += 4) {
-      float wvv[VEC];
-      load_vec<WT, VEC>(W + (size_t)k * N + c0, wvv);
-#pragma unroll
-      for (int m = 0; m < MR; m++) {
-        // rows past M (never stored) read row M - 1: no branch around the load
-        const float xm = x[(size_t)min(m, M - 1) * K + k];
-#pragma unroll
-        for (int j = 0; j < VEC; j++) acc[m][j] += xm * wvv[j];
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < MR; m++)
-#pragma unroll
-    for (int j = 0; j < VEC; j++) red[wv][m][lane * VEC + j] = acc[m][j];
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < MR * TILE; idx += 256) {
-    const int m = idx / TILE, cc = idx % TILE;
-    const int col = blockIdx.x * TILE + cc;
-    if (m < M && col < N)
-      part[((size_t)s * M + m) * N + col] = red[0][m][cc] + red[1][m][cc] + red[2][m][cc] + red[3][m][cc];
-  }
-}
-
 __global__ __launch_bounds__(256) void k_splitk_epilogue(const float* __restrict__ part, int S, int M, int N,
                                                          const float* __restrict__ bias, int epi,
                                                          const float* __restrict__ res, float* __restrict__ y) {
@@ -1442,25 +1394,6 @@ hipError_t launch_layernorm_bf16(hipStream_t st, const float* in, int rows, cons
   return hipGetLastError();
 }
 
-template <typename WT>
-hipError_t launch_gemv_splitk(hipStream_t st, const float* x, int M, int K, const WT* W, int N, float* part,
-                              int splits, int* used_splits) {
-  constexpr int VEC = 16 / sizeof(WT);
-  constexpr int TILE = 64 * VEC;
-  FH_CHECK_ARG(M >= 1 && M <= 4 && K > 0 && N > 0 && N % VEC == 0 && splits >= 1 && x && W && part);
-  const int kchunk = (K + splits - 1) / splits;
-  const int S = (K + kchunk - 1) / kchunk;
-  *used_splits = S;
-  dim3 grid((N + TILE - 1) / TILE, S);
-  if (M == 1)
-    hipLaunchKernelGGL((k_gemv_splitk<WT, 1>), grid, dim3(256), 0, st, x, M, K, W, N, kchunk, part);
-  else if (M == 2)
-    hipLaunchKernelGGL((k_gemv_splitk<WT, 2>), grid, dim3(256), 0, st, x, M, K, W, N, kchunk, part);
-  else
-    hipLaunchKernelGGL((k_gemv_splitk<WT, 4>), grid, dim3(256), 0, st, x, M, K, W, N, kchunk, part);
-  return hipGetLastError();
-}
-
 hipError_t launch_splitk_epilogue(hipStream_t st, const float* part, int splits, int M, int N, const float* bias,
                                   int epi, const float* res, float* y) {
   FH_CHECK_ARG(splits >= 1 && M > 0 && N > 0 && part && y);
@@ -1605,10 +1538,6 @@ template hipError_t launch_embed<float>(hipStream_t, RowSrc, int, int, const flo
                                               int, float*);
 template hipError_t launch_embed<bf16_t>(hipStream_t, RowSrc, int, int, const bf16_t*, const bf16_t*, int,
                                                int, int, float*);
-template hipError_t launch_gemv_splitk<float>(hipStream_t, const float*, int, int, const float*, int, float*, int,
-                                              int*);
-template hipError_t launch_gemv_splitk<bf16_t>(hipStream_t, const float*, int, int, const bf16_t*, int, float*, int,
-                                               int*);
 template hipError_t launch_gemm<float>(hipStream_t, const float*, int, int, const float*, int, const float*, int,
                                        const float*, float*);
 template hipError_t launch_gemm<bf16_t>(hipStream_t, const float*, int, int, const bf16_t*, int, const float*, int,

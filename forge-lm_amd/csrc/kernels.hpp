@@ -23,10 +23,21 @@ hipError_t launch_layernorm(hipStream_t st, const float* in, int rows, int rows_
 hipError_t launch_layernorm_bf16(hipStream_t st, const float* in, int rows, const float* w, const float* b,
                                  bf16_t* out, int d, float eps);
 
-// Split-K GEMV for M <= 4 rows: part[s][m][n] = sum_{k in chunk s} x[m,k] W[k,n].
+// Where a qkv projection's K and V columns go: the caches [..][H][ctx][hd] at pos(row), row
+// r of sequence r / T.
+template <typename KT>
+struct QkvStore {
+  RowSrc src;
+  int T, H, ctx;
+  KT* kc;
+  KT* vc;
+};
+// y = epi(LN(x) @ W + bias) (+ res) for M <= 4 rows (gemv.hip), W transposed as Wt[N][K]; K a
+// multiple of 8 up to 4096.  ln_w null: x as it is; else K <= 1024.  kv with EPI_QKV.
 template <typename WT>
-hipError_t launch_gemv_splitk(hipStream_t st, const float* x, int M, int K, const WT* W, int N, float* part,
-                              int splits, int* used_splits);
+hipError_t launch_gemv(hipStream_t st, const float* x, int M, int K, const WT* Wt, int N, const float* ln_w,
+                       const float* ln_b, float eps, const float* bias, int epi, const float* res, float* y,
+                       const QkvStore<WT>* kv = nullptr);
 
 // y[m,n] = epi(sum_s part[s][m][n] + bias[n]) (+ res[m,n]).
 hipError_t launch_splitk_epilogue(hipStream_t st, const float* part, int splits, int M, int N, const float* bias,
@@ -103,6 +114,12 @@ template <typename KT>
 hipError_t launch_attn_decode_wide(hipStream_t st, RowSrc src, const float* qkv, int B, int d, int H, int ctx,
                                    const KT* kcache, const KT* vcache, float* part, float* o, bool combine = true,
                                    const QkvParts* qp = nullptr);
+
+// The same for caches of at most 256 positions, in one launch (attn_decode_one_fits).
+bool attn_decode_one_fits(int d, int H, int ctx, int esize);
+template <typename KT>
+hipError_t launch_attn_decode_one(hipStream_t st, RowSrc src, const float* qkv, int B, int d, int H, int ctx,
+                                  const KT* kc, const KT* vc, float* o);
 
 // Tied head for B rows: logits[b, v] = dot(xn[b,:], E[v,:]).
 template <typename WT>

@@ -1168,3 +1168,31 @@ def test_each_path_gives_the_same_bits_run_to_run(fhp, oracle, backend, path):
                                   np.asarray(first[1], np.float32).view(np.uint32)), path
     for m in models:
         m.dispose()
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("ctx,D,H", [(40, 8, 2), (256, 40, 2), (257, 40, 2), (130, 200, 5), (256, 128, 2), (64, 1024, 16),
+                                     (60, 96, 1)])
+def test_few_row_decode_shapes_match_oracle(fhp, oracle, backend, B, ctx, D, H):
+    """Decode steps of up to 4 rows (GEMVs with their LayerNorms, the one-launch attention up to 256
+    positions) and just past them: widths that fill a lane's pieces or not, K over one wave and over
+    four, head widths 4 to 96, an odd vocabulary."""
+    m, oc, w = make_model(fhp, oracle, backend, (131, ctx, D, 2, H), 7 + D, batch=B)
+    prompts = np.stack([fhp.TrainingRandom(90 + b).ids(131, 5) for b in range(B)])
+    ids, lg = fhp.Sampler.generate(m, prompts, 12, 0.0, 0, None, return_logits=True)
+    m.dispose()
+    for b in range(B):
+        rids, rlg = oracle.generate(oc, w, prompts[b], 12, return_logits=True)
+        assert_greedy_parity(ids[b], lg[b], rids, rlg, TOL_F32, f"sequence {b}")
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (2, 2), (1, 4), (1, 5), (4, 8), (3, 11), (1, 64), (5, 13)])
+def test_window_row_counts_match_oracle(fhp, oracle, backend, B, T):
+    """fp32 windows at the row counts that change kernels (4, 32 and 64 rows in all)."""
+    m, oc, w = make_model(fhp, oracle, backend, (131, 64, 64, 2, 2), 3, batch=B)
+    ids = np.stack([fhp.TrainingRandom(7 + b).ids(131, T) for b in range(B)])
+    got = m.forward_last(ids)
+    m.dispose()
+    for b in range(B):
+        _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
+        assert rel_err(got[b], rlg[0]) <= TOL_F32
