@@ -265,6 +265,136 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const QT* __restrict_
 }
 
 // ---------------------------------------------------------------------------
+// fp32 windows: 32 queries of one (sequence, head) per block, whose four waves take every
+// fourth key tile and merge their softmax sums through LDS at the end.  The fp32 MFMAs are the
+// work (64 cycles each, 128 per tile), so what counts is how many waves share it: blocks of 128
+// queries put 36 of them on 256 CUs for 12 heads of 333 rows.  The waves share nothing until the
+// merge, so K and V go from L2 straight into registers, in the operand layout: lanes l and
+// l + 32 hold dims 0-31 and 32-63 of key row l (the products of a step are summed whatever
+// dims it pairs), and a V step reads 32 dims of two keys.  No LDS tile, no barrier per tile.
+constexpr int KQ = 32;  // queries per block
+__global__ __launch_bounds__(256, 2) void k_attn_prefill_keys(const float* __restrict__ qp, int qstride, int T, int d,
+                                                              int H, int ctx, const float* __restrict__ kc,
+                                                              const float* __restrict__ vc, float* __restrict__ o) {
+  __shared__ float om[4][KQ], ol[4][KQ];
+  __shared__ float os[4][KQ][HD + 1];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nqb = (T + KQ - 1) / KQ;
+  const QBlock qbk = prefill_block(blockIdx.x, nqb, H);
+  const int t0 = (nqb - 1 - qbk.qb) * KQ, h = qbk.h, b = qbk.b;
+  const int col = lane & 31, half = lane >> 5, q = t0 + col;
+  const float scale = 0.125f;  // 1 / sqrt(64), exact
+  const size_t head = ((size_t)b * H + h) * ctx * HD;
+  const __amdgpu_buffer_rsrc_t rk =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(kc + head), (short)0, T * HD * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(vc + head), (short)0, T * HD * 4, 0x00020000);
+  const float* qrow = qp + (size_t)(b * T + min(q, T - 1)) * qstride + h * HD + 32 * half;
+  float qf[32];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float4 a = *reinterpret_cast<const float4*>(qrow + 4 * i);
+    qf[4 * i] = a.x, qf[4 * i + 1] = a.y, qf[4 * i + 2] = a.z, qf[4 * i + 3] = a.w;
+  }
+  f32x16_t ot[2];  // O^T: dims (dt * 32 + acc_row) x this lane's query
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) ot[dt][r] = 0.f;
+  float m = -INFINITY, l = 0.f;
+
+  const int nkt = (min(t0 + KQ, T) - 1) / BKV + 1;
+  for (int kt = w; kt < nkt; kt += 4) {
+    const int k0 = kt * BKV;
+    // rows at or past T read as zeros
+    u32x4_t kr[2][8];
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        kr[jt][i] =
+            __builtin_amdgcn_raw_buffer_load_b128(rk, ((k0 + jt * 32 + col) * HD + 32 * half + 4 * i) * 4, 0, 0);
+    float vr[2][16][2];  // [key half][score register][dim half]
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+          vr[jt][r][dt] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              rv, ((k0 + jt * 32 + acc_row(lane, r)) * HD + dt * 32 + col) * 4, 0, 0));
+    f32x16_t s[2];
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) s[jt][r] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+          s[jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[jt][i][j]), qf[4 * i + j], s[jt], 0, 0, 0);
+    float mt = -INFINITY;
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int key = k0 + jt * 32 + acc_row(lane, r);
+        s[jt][r] = key <= q && key < T ? s[jt][r] * scale : -INFINITY;
+        mt = fmaxf(mt, s[jt][r]);
+      }
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float mn = fmaxf(m, mt);
+    const float corr = m == -INFINITY ? 0.f : expf(m - mn);
+    float ls = 0.f;
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const float p = s[jt][r] == -INFINITY ? 0.f : expf(s[jt][r] - mn);
+        s[jt][r] = p;
+        ls += p;
+      }
+    ls += __shfl_xor(ls, 32, 64);
+    l = l * corr + ls;
+    m = mn;
+#pragma unroll
+    for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) ot[dt][r] *= corr;
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+      for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int dt = 0; dt < 2; dt++)
+          ot[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[jt][r][dt], s[jt][r], ot[dt], 0, 0, 0);
+  }
+
+  // merge: each wave's sums at the block's maximum (a query's first key is in tile 0, so that
+  // maximum is a score; a wave without a key of the query has m = -inf and contributes 0)
+  if (half == 0) om[w][col] = m;
+  __syncthreads();
+  const float mx = fmaxf(fmaxf(om[0][col], om[1][col]), fmaxf(om[2][col], om[3][col]));
+  const float f = m == -INFINITY ? 0.f : expf(m - mx);
+  if (half == 0) ol[w][col] = l * f;
+#pragma unroll
+  for (int dt = 0; dt < 2; dt++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) os[w][col][dt * 32 + acc_row(lane, r)] = ot[dt][r] * f;
+  __syncthreads();
+  for (int e = tid; e < KQ * HD; e += 256) {
+    const int qq = e / HD, dim = e % HD;
+    if (t0 + qq >= T) break;
+    const float sum = ol[0][qq] + ol[1][qq] + ol[2][qq] + ol[3][qq];
+    o[(size_t)(b * T + t0 + qq) * d + h * HD + dim] =
+        (os[0][qq][dim] + os[1][qq][dim] + os[2][qq][dim] + os[3][qq][dim]) / sum;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // bf16 sessions with q already in bf16: the same S^T / O^T scheme, software-
 // pipelined.  The K and V^T tiles of key tile j + 1 are fetched into registers
 // while tile j is multiplied and land in the other half of a double-buffered
@@ -449,7 +579,19 @@ hipError_t launch_attn_prefill_mfma(hipStream_t st, const float* qkv, int B, int
   if (B <= 0 || T <= 0 || T > ctx || H <= 0 || d != H * HD || !qkv || !kcache || !vcache || !o ||
       (size_t)T * HD * sizeof(KT) > 0x7fffffffu)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_prefill_mfma<KT, OT, float>), dim3((T + BQ - 1) / BQ * H * B), dim3(256), 0, st, qkv,
+  const int blocks = (T + BQ - 1) / BQ * H * B;
+  if constexpr (sizeof(KT) == 4) {
+    // below two 128-query blocks per CU the waves are too few (ms per forward of the 98M shape,
+    // 128-query blocks against 32-query ones: 333 rows 1.68 / 1.42, 1024 rows 2.92 / 2.34, 3 x 700
+    // 3.75 / 3.54, 16 x 200 4.33 / 4.31); above, sharing a K/V tile in LDS wins (8 x 1024 10.4 /
+    // 10.6, 32 x 512 17.2 / 17.6)
+    if (blocks <= 512) {
+      hipLaunchKernelGGL(k_attn_prefill_keys, dim3((T + KQ - 1) / KQ * H * B), dim3(256), 0, st, qkv, 3 * d, T, d, H,
+                         ctx, kcache, vcache, o);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((k_attn_prefill_mfma<KT, OT, float>), dim3(blocks), dim3(256), 0, st, qkv,
                      3 * d, T, d, H, ctx, kcache, vcache, o);
   return hipGetLastError();
 }

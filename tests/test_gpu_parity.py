@@ -1196,3 +1196,16 @@ def test_window_row_counts_match_oracle(fhp, oracle, backend, B, T):
     for b in range(B):
         _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
         assert rel_err(got[b], rlg[0]) <= TOL_F32
+
+
+@pytest.mark.parametrize("B,T", [(1, 31), (1, 33), (2, 64), (1, 65), (1, 129), (3, 257), (130, 20), (65, 150)])
+def test_fp32_window_attention_blocks_match_oracle(fhp, oracle, backend, B, T):
+    """head_dim 64 windows in fp32 at the edges of the 32-query blocks and their 64-key tiles, with one to
+    five tiles over the four waves, and on both sides of the block count that picks 128-query blocks."""
+    m, oc, w = make_model(fhp, oracle, backend, (67, 300, 256, 2, 4), 5, batch=B)
+    ids = np.stack([fhp.TrainingRandom(300 + b).ids(67, T) for b in range(B)])
+    got = m.forward_last(ids)
+    m.dispose()
+    for b in sorted({0, B // 2, B - 1}):
+        _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
+        assert rel_err(got[b], rlg[0]) <= TOL_F32
