@@ -360,15 +360,17 @@ size_t split_blocks(int bm, int bn, int slots, int M, int N) {
   return (size_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * slots;
 }
 
-// Tile and K splits by a cost in microseconds that was fitted to a sweep of tiles and
-// splits over products of 64 .. 8192 rows (each plan's estimate within 15% of its time):
-// a CU runs its blocks' stages at 1.2 / 0.7 / 0.42 us each for the three tiles (a large
-// tile does the most per operand byte: 217 / 190 / 168 TFLOP/s at 8192 x 4096 x 4096) and a
-// lone block no faster than one load round trip per stage; splitting K costs the partial
-// sums' way through memory and a second launch.  2048 x 3072 x 768: 128 x 128 tiles in 8
-// splits 64 us, unsplit 109.
+// Tile and K splits by a cost in microseconds, fitted to the times of every tile and split over
+// 84 products (40 .. 16257 rows, K 64 .. 16257, plain and batched; weights cold): what it picks
+// is 1.8% off the fastest in the geometric mean and 11% at worst.  A launch costs `fixed`, and
+// `round` more per round of blocks over the CUs; a stage costs a CU `unit` per block of its own
+// (a large tile does the most per operand byte: 217 / 190 / 168 TFLOP/s at 8192 x 4096 x 4096),
+// a lone block no less than `alone` (its chain of load, split, LDS and MFMAs); splitting K costs a
+// second launch and the partial sums' way through memory.  2048 x 3072 x 768: 128 x 128 tiles in
+// 8 splits 64 us, unsplit 109; 100 x 768 x 768: 64 x 64 in 8 splits 9.5, unsplit 23.
 SplitPlan split_plan(int slots, int M, int K, int N, size_t part_floats, int cus) {
-  constexpr double unit[3] = {1.2, 0.7, 0.42}, alone[3] = {1.35, 1.0, 0.8};
+  constexpr double fixed[3] = {4.6, 3.9, 4.1}, round[3] = {1.5, 0.7, 0.24};
+  constexpr double alone[3] = {1.78, 1.2, 0.77}, unit[3] = {1.17, 0.74, 0.45};
   constexpr int counts[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
   const double mn = (double)slots * M * N;
   SplitPlan best{64, 64, 1};
@@ -379,8 +381,8 @@ SplitPlan split_plan(int slots, int M, int K, int N, size_t part_floats, int cus
       if (S > 1 && (K < S * 2 * SK || mn * S > (double)part_floats)) break;
       const double rounds = (double)(((size_t)tiles * S + cus - 1) / cus);
       const int stages = ((K + S - 1) / S + SK - 1) / SK;
-      double us = 3.0 + stages * std::max(alone[i], rounds * unit[i]);
-      if (S > 1) us += 3.0 + mn * (S + 1) * 4 / 3.5e6;
+      double us = fixed[i] + rounds * round[i] + stages * std::max(alone[i], rounds * unit[i]);
+      if (S > 1) us += 2.8 + mn * (S + 1) * 4 / 5.2e6;
       if (us < best_us) {
         best_us = us;
         best = SplitPlan{kTiles[i][0], kTiles[i][1], S};
