@@ -511,6 +511,7 @@ constexpr int kST = 1024;        // sampler block size
 constexpr int kMaxVocab = 65536; // LDS bitmaps hold V bits
 constexpr int kSurvCap = 4096;   // top-k survivors summed in index order
 constexpr int kRowV = 16;        // logits per thread in the register sampler (V <= kST * kRowV)
+constexpr int kRankKeys = 256;   // candidates ranked against each other (more: radix passes)
 
 __device__ __forceinline__ uint32_t order_key(float f) {
   uint32_t u = __float_as_uint(f);
@@ -661,8 +662,8 @@ struct SampleRowSmem {
   int redi[2][kST / 64];
   int cntp[2][kST / 64][2];
   int wscan[kST / 64];
-  uint32_t ckey[1024];
-  int ladder[8][kST / 64];
+  alignas(16) uint32_t ckey[1024];
+  alignas(16) int ladder[8][kST / 64];
   int surv[kSurvCap];
   float survv[kSurvCap];
   float part[kST];
@@ -671,13 +672,25 @@ struct SampleRowSmem {
 
 // block max of one value per thread (all threads get it); slot alternates between calls
 __device__ __forceinline__ float row_block_max(float v, SampleRowSmem& sm, int slot) {
-  v = wave_max(v);
+  v = wave_max_dpp(v);
   if ((threadIdx.x & 63) == 0) sm.redf[slot][threadIdx.x >> 6] = v;
   __syncthreads();
   float r = sm.redf[slot][0];
 #pragma unroll
   for (int i = 1; i < kST / 64; i++) r = fmaxf(r, sm.redf[slot][i]);
   return r;
+}
+
+// smallest of a wave's ints (DPP row operations, as wave_sum_dpp)
+__device__ __forceinline__ int wave_min_int_dpp(int v) {
+  constexpr int big = 0x7fffffff;
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0xB1, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0x4E, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0x141, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0x140, 0xF, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0x142, 0xA, 0xF, false));
+  v = min(v, __builtin_amdgcn_update_dpp(big, v, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(v, 63);
 }
 
 __device__ __forceinline__ int row_block_argmax(const float (&x)[kRowV], int V, SampleRowSmem& sm, int slot) {
@@ -688,7 +701,10 @@ __device__ __forceinline__ int row_block_argmax(const float (&x)[kRowV], int V, 
     const int i = threadIdx.x * kRowV + j;
     if (i < V) argmax_merge(best, bi, x[j], i);
   }
-  wave_argmax(best, bi);
+  // the wave's largest, then the smallest index that holds it (what argmax_merge keeps)
+  const float wbest = wave_max_dpp(best);
+  bi = wave_min_int_dpp(best == wbest ? bi : 0x7fffffff);
+  best = wbest;
   if ((threadIdx.x & 63) == 0) {
     sm.redf[slot][threadIdx.x >> 6] = best;
     sm.redi[slot][threadIdx.x >> 6] = bi;
@@ -713,16 +729,25 @@ __global__ __launch_bounds__(kST) void k_sample_row(SampleArgs a) {
   if (a.dump && n < a.max_new)
     for (int i = tid; i < V; i += kST) a.dump[((size_t)b * a.max_new + n) * V + i] = lg[i];
   float x[kRowV];
-  if ((V & 3) == 0 && (reinterpret_cast<uintptr_t>(lg) & 15) == 0) {
-    // 16-byte loads; groups past V load the last group and drop it (no branch around the loads)
+  if (V >= 4) {
+    // 16-byte loads, at 4-byte alignment (rows of an odd V, any caller's row: 16 strided 4-byte
+    // loads per thread took 6 us at V 16257); a group that passes V loads the row's last four and
+    // takes its own from them, with no branch around the loads
+    struct __attribute__((packed, aligned(4))) Quad {
+      float v[4];
+    };
 #pragma unroll
     for (int q = 0; q < kRowV / 4; q++) {
-      const int i = tid * kRowV + 4 * q;
-      const float4 v = *reinterpret_cast<const float4*>(lg + min(i, V - 4));
-      x[4 * q] = v.x;
-      x[4 * q + 1] = v.y;
-      x[4 * q + 2] = v.z;
-      x[4 * q + 3] = v.w;
+      const int i = tid * kRowV + 4 * q, at = min(i, V - 4), sh = i - at;
+      const Quad f = *reinterpret_cast<const Quad*>(lg + at);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float v = f.v[j];  // sh == 0, but for the last groups
+#pragma unroll
+        for (int t = 1; t < 4; t++)
+          if (j + t < 4) v = sh == t ? f.v[j + t] : v;
+        x[4 * q + j] = v;
+      }
     }
   } else {
 #pragma unroll
@@ -845,11 +870,17 @@ __global__ __launch_bounds__(kST) void k_sample_row(SampleArgs a) {
               if (lane == 0) sm.ladder[q][wv] = cl[q];
             }
             __syncthreads();
+            // the waves' counts added up by every wave: 8 lanes to a window, two counts to a lane
+            const int2 lc = *reinterpret_cast<const int2*>(&sm.ladder[lane >> 3][2 * (lane & 7)]);
+            int tot8 = lc.x + lc.y;
+            tot8 += __builtin_amdgcn_update_dpp(0, tot8, 0xB1, 0xF, 0xF, false);
+            tot8 += __builtin_amdgcn_update_dpp(0, tot8, 0x4E, 0xF, 0xF, false);
+            tot8 += __builtin_amdgcn_update_dpp(0, tot8, 0x141, 0xF, 0xF, false);
             int pick = -1;
-            for (int q = 0; q < 8 && pick < 0; q++) {
-              int tot = 0;
-              for (int w2 = 0; w2 < kST / 64; w2++) tot += sm.ladder[q][w2];
-              if (tot >= a.top_k) pick = tot <= 1024 ? q : 8;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+              const int tot = __builtin_amdgcn_readlane(tot8, 8 * q);
+              if (pick < 0 && tot >= a.top_k) pick = tot <= 1024 ? q : 8;
             }
             if (pick >= 0 && pick < 8) lo = M - (float)(1 << pick) * 0.125f;
           }
@@ -930,7 +961,24 @@ __global__ __launch_bounds__(kST) void k_sample_row(SampleArgs a) {
             if ((key[j] & hm) == prefix) sm.ckey[off++] = key[j];
           __syncthreads();
         }
-        if (sh >= 0) {
+        if (sh >= 0 && nin <= kRankKeys) {
+          // few keys: the k-th largest is the one that fewer than k others beat, equal ones in
+          // list order (thread t ranks key t against all of them, four to an LDS read)
+          if (tid < kRankKeys && tid >= nin) sm.ckey[tid] = 0u;
+          __syncthreads();
+          if (tid < nin) {
+            const uint32_t mine = sm.ckey[tid];
+            int rank = 0;
+            for (int i = 0; i < nin; i += 4) {
+              const uint4 o = *reinterpret_cast<const uint4*>(&sm.ckey[i]);
+              rank += (o.x > mine || (o.x == mine && i < tid)) + (o.y > mine || (o.y == mine && i + 1 < tid)) +
+                      (o.z > mine || (o.z == mine && i + 2 < tid)) + (o.w > mine || (o.w == mine && i + 3 < tid));
+            }
+            if (rank == rem - 1) sm.misc[1] = (int)mine;
+          }
+          __syncthreads();
+          prefix = (uint32_t)sm.misc[1];
+        } else if (sh >= 0) {
           if (wv == 0) {
             constexpr int E = 1024 / 64;
             const int ne = (nin + 63) >> 6;  // filled key groups (uniform)
@@ -1033,7 +1081,7 @@ __global__ __launch_bounds__(kST) void k_sample_row(SampleArgs a) {
           for (int c0 = 0; c0 < nsurv; c0 += 64) {
             const float e = (c0 + lane < nsurv) ? expf(sm.survv[c0 + lane] - mx) : 0.f;
             const int m = min(64, nsurv - c0);
-            for (int q = 0; q < m; q++) sum = sum + __shfl(e, q, 64);
+            for (int q = 0; q < m; q++) sum = sum + lane_bcast(e, q);
           }
           const float u = (float)u01 * sum;
           float acc = 0.f;
@@ -1043,7 +1091,7 @@ __global__ __launch_bounds__(kST) void k_sample_row(SampleArgs a) {
             const float e = (c0 + lane < nsurv) ? expf(sm.survv[c0 + lane] - mx) : 0.f;
             const int m = min(64, nsurv - c0);
             for (int q = 0; q < m; q++) {
-              acc = acc + __shfl(e, q, 64);
+              acc = acc + lane_bcast(e, q);
               if (u < acc) {
                 r = sm.surv[c0 + q];
                 found = true;

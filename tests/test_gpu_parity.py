@@ -265,6 +265,28 @@ def test_sampler_top_k_selection(fhp, oracle, backend, shape, k):
     dev.free()
 
 
+@pytest.mark.parametrize("V", [1, 3, 4, 5, 15, 17, 1023, 4099, 16257, 16383])
+@pytest.mark.parametrize("k", [1, 40, 255, 256, 257, 900])
+def test_sampler_row_widths_and_candidate_counts(fhp, oracle, backend, V, k):
+    """Rows that end inside a 16-byte group or are shorter than one, at a row address 4 bytes past a
+    multiple of 16 too, and candidate counts on both sides of the 256 that are ranked directly, with ties
+    among them: the device id equals the oracle's, greedy and sampled."""
+    rng = np.random.default_rng(V * 1000 + k)
+    for step in (0.0, 0.25):  # 0.25: values on a grid, so that many tie
+        lg = rng.standard_normal(V + 1).astype(np.float32) * 2
+        if step:
+            lg = np.round(lg / step).astype(np.float32) * np.float32(step)
+        dev = fhp.DeviceBuffer.from_array(backend, lg)
+        for first in (0, 1):
+            row = lg[first:first + V]
+            ptr = dev.ptr.value + 4 * first
+            assert fhp.Sampler.sample_device_logits(backend, ptr, V, [], 0.0, 0, 0.0) == int(np.argmax(row))
+            for u in (0.0, 0.6, 0.9999):
+                got = fhp.Sampler.sample_device_logits(backend, ptr, V, [], 0.9, k, u)
+                assert got == oracle.sample(row, 0.9, k, u), (step, first, u)
+        dev.free()
+
+
 def decision_gaps(adj, T, k, u):
     """How far Sampler.Sample's decision (Sampler.cs:29-69) on the adjusted logits
     `adj` is from changing: (top-k gap, CDF gap).  The top-k gap is the distance
