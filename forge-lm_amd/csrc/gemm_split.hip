@@ -48,9 +48,11 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
-// 16-byte chunk c of row r is stored at chunk c ^ bits 2-3 of r: eight lanes that read
-// (or write) the same chunk of eight consecutive rows touch different banks
-__device__ __forceinline__ int split_swz(int r, int c) { return c ^ ((r >> 2) & 3); }
+// 16-byte chunk c of row r is stored at chunk c ^ g(r), with g different over rows r, r + 4,
+// r + 8, r + 12 (16 rows of one chunk fill the 64 banks that reads see) and over pairs of rows (8 rows
+// fill the 32 that writes see): no bank conflicts either way.  bits 2-3 of r alone cost the
+// row-contiguous operands 5% of the CU's cycles each in write conflicts.
+__device__ __forceinline__ int split_swz(int r, int c) { return c ^ (((r >> 1) ^ (r >> 3 & 1)) & 3); }
 
 // two elements -> their three bf16 parts, packed (round to nearest even at each step;
 // the subtractions are exact)
@@ -361,8 +363,8 @@ size_t split_blocks(int bm, int bn, int slots, int M, int N) {
 }
 
 // Tile and K splits by a cost in microseconds, fitted to the times of every tile and split over
-// 84 products (40 .. 16257 rows, K 64 .. 16257, plain and batched; weights cold): what it picks
-// is 1.8% off the fastest in the geometric mean and 11% at worst.  A launch costs `fixed`, and
+// 92 products (40 .. 16257 rows, K 64 .. 16257, plain and batched; weights cold): what it picks
+// is 1.4% off the fastest in the geometric mean and 10% at worst.  A launch costs `fixed`, and
 // `round` more per round of blocks over the CUs; a stage costs a CU `unit` per block of its own
 // (a large tile does the most per operand byte: 217 / 190 / 168 TFLOP/s at 8192 x 4096 x 4096),
 // a lone block no less than `alone` (its chain of load, split, LDS and MFMAs); splitting K costs a
@@ -371,7 +373,7 @@ size_t split_blocks(int bm, int bn, int slots, int M, int N) {
 SplitPlan split_plan(int slots, int M, int K, int N, size_t part_floats, int cus) {
   constexpr double fixed[3] = {4.6, 3.9, 4.1}, round[3] = {1.5, 0.7, 0.24};
   constexpr double alone[3] = {1.78, 1.2, 0.77}, unit[3] = {1.17, 0.74, 0.45};
-  constexpr int counts[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+  constexpr int counts[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32};
   const double mn = (double)slots * M * N;
   SplitPlan best{64, 64, 1};
   double best_us = 1e300;
