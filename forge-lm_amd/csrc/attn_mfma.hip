@@ -267,12 +267,13 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const QT* __restrict_
 // ---------------------------------------------------------------------------
 // fp32 windows: 32 queries of one (sequence, head) per block, whose four waves take every
 // fourth key tile and merge their softmax sums through LDS at the end.  The fp32 MFMAs are the
-// work (64 cycles each, 128 per tile), so what counts is how many waves share it: blocks of 128
+// work (64 cycles each, 64 per 32-key tile), so what counts is how many waves share it: blocks of 128
 // queries put 36 of them on 256 CUs for 12 heads of 333 rows.  The waves share nothing until the
 // merge, so K and V go from L2 straight into registers, in the operand layout: lanes l and
 // l + 32 hold dims 0-31 and 32-63 of key row l (the products of a step are summed whatever
 // dims it pairs), and a V step reads 32 dims of two keys.  No LDS tile, no barrier per tile.
-constexpr int KQ = 32;  // queries per block
+constexpr int KQ = 32;   // queries per block
+constexpr int KKV = 32;  // keys per tile
 __global__ __launch_bounds__(256, 2) void k_attn_prefill_keys(const float* __restrict__ qp, int qstride, int T, int d,
                                                               int H, int ctx, const float* __restrict__ kc,
                                                               const float* __restrict__ vc, float* __restrict__ o) {
@@ -303,60 +304,48 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_keys(const float* __res
     for (int r = 0; r < 16; r++) ot[dt][r] = 0.f;
   float m = -INFINITY, l = 0.f;
 
-  const int nkt = (min(t0 + KQ, T) - 1) / BKV + 1;
+  const int nkt = (min(t0 + KQ, T) - 1) / KKV + 1;
   for (int kt = w; kt < nkt; kt += 4) {
-    const int k0 = kt * BKV;
+    const int k0 = kt * KKV;
     // rows at or past T read as zeros
-    u32x4_t kr[2][8];
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-      for (int i = 0; i < 8; i++)
-        kr[jt][i] =
-            __builtin_amdgcn_raw_buffer_load_b128(rk, ((k0 + jt * 32 + col) * HD + 32 * half + 4 * i) * 4, 0, 0);
-    float vr[2][16][2];  // [key half][score register][dim half]
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++)
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-          vr[jt][r][dt] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-              rv, ((k0 + jt * 32 + acc_row(lane, r)) * HD + dt * 32 + col) * 4, 0, 0));
-    f32x16_t s[2];
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) s[jt][r] = 0.f;
-    }
+    u32x4_t kr[8];
 #pragma unroll
     for (int i = 0; i < 8; i++)
+      kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, ((k0 + col) * HD + 32 * half + 4 * i) * 4, 0, 0);
+    float vr[16][2];  // [score register][dim half]
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+    for (int r = 0; r < 16; r++)
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++)
-          s[jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[jt][i][j]), qf[4 * i + j], s[jt], 0, 0, 0);
+      for (int dt = 0; dt < 2; dt++)
+        vr[r][dt] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rv, ((k0 + acc_row(lane, r)) * HD + dt * 32 + col) * 4, 0, 0));
+    // two accumulators: one would be a single chain of 32 dependent MFMAs
+    f32x16_t s, s2;
+#pragma unroll
+    for (int r = 0; r < 16; r++) s[r] = s2[r] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[i][0]), qf[4 * i], s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[i][1]), qf[4 * i + 1], s2, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[i][2]), qf[4 * i + 2], s, 0, 0, 0);
+      s2 = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(kr[i][3]), qf[4 * i + 3], s2, 0, 0, 0);
+    }
     float mt = -INFINITY;
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int key = k0 + jt * 32 + acc_row(lane, r);
-        s[jt][r] = key <= q && key < T ? s[jt][r] * scale : -INFINITY;
-        mt = fmaxf(mt, s[jt][r]);
-      }
+    for (int r = 0; r < 16; r++) {
+      const int key = k0 + acc_row(lane, r);
+      s[r] = key <= q && key < T ? (s[r] + s2[r]) * scale : -INFINITY;
+      mt = fmaxf(mt, s[r]);
+    }
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
     const float mn = fmaxf(m, mt);
     const float corr = m == -INFINITY ? 0.f : expf(m - mn);
     float ls = 0.f;
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const float p = s[jt][r] == -INFINITY ? 0.f : expf(s[jt][r] - mn);
-        s[jt][r] = p;
-        ls += p;
-      }
+    for (int r = 0; r < 16; r++) {
+      s[r] = s[r] == -INFINITY ? 0.f : expf(s[r] - mn);
+      ls += s[r];
+    }
     ls += __shfl_xor(ls, 32, 64);
     l = l * corr + ls;
     m = mn;
@@ -365,12 +354,10 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_keys(const float* __res
 #pragma unroll
       for (int r = 0; r < 16; r++) ot[dt][r] *= corr;
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
+    for (int r = 0; r < 16; r++)
 #pragma unroll
-      for (int r = 0; r < 16; r++)
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-          ot[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[jt][r][dt], s[jt][r], ot[dt], 0, 0, 0);
+      for (int dt = 0; dt < 2; dt++)
+        ot[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[r][dt], s[r], ot[dt], 0, 0, 0);
   }
 
   // merge: each wave's sums at the block's maximum (a query's first key is in tile 0, so that
