@@ -571,11 +571,12 @@ __global__ void k_embedding_forward(const float* __restrict__ table, const int* 
 }
 
 // dTable[id] += dOut[t] for the positions t of each distinct id, in ascending order (the CPU
-// loop's sums).  Block t works if no earlier position has its id: it lists the later ones that
-// do in LDS, in order, and each thread adds up its columns with 8 loads in flight (a text's
-// commonest token comes up often: 80 of 2048 positions one load at a time took 15 us).  The ids
-// are compared n^2 times in all, 16 to a thread at n = 2048; up to kScatterIds positions that is
-// less than sorting them on the host took.
+// loop's sums).  Block t works if no earlier position has its id: each thread compares a
+// run of positions, a scan over the threads lists the later ones that match in LDS in order, and
+// each thread adds up four columns at a time with 8 loads of each in flight (a text's commonest token
+// comes up often: 80 of 2048 positions, one load at a time, took 15 us).  The ids are compared n^2
+// times in all, 8 to a thread at n = 2048; up to kScatterIds positions that is less than sorting
+// them on the host took.
 constexpr int kScatterIds = 8192;
 __global__ __launch_bounds__(256) void k_embedding_scatter(const float* __restrict__ dout, const int* __restrict__ idx,
                                                            int n, float* __restrict__ dtable, int D) {
@@ -583,35 +584,56 @@ __global__ __launch_bounds__(256) void k_embedding_scatter(const float* __restri
   __shared__ int counts[4];
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int id = idx[t];
-  int dup = 0;
-  for (int j = tid; j < t; j += 256) dup |= idx[j] == id;
-  if (__syncthreads_or(dup)) return;
-  int m = 0;  // listed so far
-  for (int j0 = t; j0 < n; j0 += 256) {
-    const bool hit = j0 + tid < n && idx[min(j0 + tid, n - 1)] == id;
-    const unsigned long long mask = __ballot(hit);
-    if (lane == 0) counts[w] = __popcll(mask);
-    __syncthreads();
-    int at = m + __popcll(mask & ((1ull << lane) - 1));
-    for (int i = 0; i < 4; i++) {
-      if (i < w) at += counts[i];
-      m += counts[i];
-    }
-    if (hit) list[at] = j0 + tid;
-    __syncthreads();
+  constexpr int R = kScatterIds / 256;
+  const int run = (n + 255) / 256, j0 = tid * run, j1 = min(n, j0 + run);
+  unsigned hits = 0;  // bit i: position j0 + i matches
+#pragma unroll 8
+  for (int i = 0; i < run; i++) hits |= (idx[min(j0 + i, n - 1)] == id && j0 + i < j1 ? 1u : 0u) << i;
+  static_assert(R <= 32, "a run's matches fit a word");
+  const unsigned before = t <= j0 ? 0u : t - j0 >= 32 ? ~0u : (1u << (t - j0)) - 1u;  // positions below t
+  if (__syncthreads_or((hits & before) != 0)) return;
+  const int cnt = __popc(hits);
+  int incl = cnt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
   }
-  for (int c = tid; c < D; c += 256) {
-    float s = dtable[(size_t)id * D + c];
+  if (lane == 63) counts[w] = incl;
+  __syncthreads();
+  int at = incl - cnt, m = 0;
+  for (int i = 0; i < 4; i++) {
+    if (i < w) at += counts[i];
+    m += counts[i];
+  }
+  for (unsigned h = hits; h; h &= h - 1) list[at++] = j0 + __ffs(h) - 1;
+  __syncthreads();
+  for (int c0 = 0; c0 < D; c0 += 1024) {
+    float s[4];
+    int c[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      c[u] = min(c0 + tid + 256 * u, D - 1);  // columns past D repeat the last one and are not stored
+      s[u] = dtable[(size_t)id * D + c[u]];
+    }
     int k = 0;
     for (; k + 8 <= m; k += 8) {
-      float v[8];
+      float v[8][4];
 #pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = dout[(size_t)list[k + i] * D + c];
+      for (int i = 0; i < 8; i++)
 #pragma unroll
-      for (int i = 0; i < 8; i++) s = s + v[i];
+        for (int u = 0; u < 4; u++) v[i][u] = dout[(size_t)list[k + i] * D + c[u]];
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] = s[u] + v[i][u];
     }
-    for (; k < m; k++) s = s + dout[(size_t)list[k] * D + c];
-    dtable[(size_t)id * D + c] = s;
+    for (; k < m; k++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = s[u] + dout[(size_t)list[k] * D + c[u]];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (c0 + tid + 256 * u < D) dtable[(size_t)id * D + c[u]] = s[u];
   }
 }
 
