@@ -812,19 +812,45 @@ __global__ __launch_bounds__(256) void k_sum_doubles(const double* __restrict__ 
   if (threadIdx.x == 0) out[0] = s;
 }
 
-__global__ void k_adamw(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                        float* __restrict__ v, size_t n, float lr, float b1, float b2, float eps, float wd, float bc1,
-                        float bc2, int decay) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    float wi = w[i];
+// HBM-bound: 16 bytes read and 12 written per element, V (4 where the pointers are multiples of
+// 16 bytes, the last n % 4 by one) to a load.  The wide form streams past the caches (every byte is
+// used once; what stays in them is what the next pass reads, such as the gradients for their norm):
+// the norm and the update of 20.5M elements 194 -> 178 us; 4 floats to a load alone gained nothing.
+template <int V>
+__global__ __launch_bounds__(256) void k_adamw(float* __restrict__ w, const float* __restrict__ g,
+                                               float* __restrict__ m, float* __restrict__ v, size_t n, float lr,
+                                               float b1, float b2, float eps, float wd, float bc1, float bc2,
+                                               int decay) {
+  auto step = [&](float gi, float& mi, float& vi, float& wi) {
+    mi = b1 * mi + (1.f - b1) * gi;
+    vi = b2 * vi + (1.f - b2) * gi * gi;
     if (decay) wi = wi - lr * wd * wi;
     const float mh = mi / bc1, vh = vi / bc2;
-    w[i] = wi - lr * mh / (sqrtf(vh) + eps);
+    wi = wi - lr * mh / (sqrtf(vh) + eps);
+  };
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n / V; i += (size_t)gridDim.x * 256) {
+    if constexpr (V == 4) {
+      typedef float f4 __attribute__((ext_vector_type(4)));
+      const f4 gv = __builtin_nontemporal_load(reinterpret_cast<const f4*>(g) + i);
+      f4 mv = __builtin_nontemporal_load(reinterpret_cast<f4*>(m) + i);
+      f4 vv = __builtin_nontemporal_load(reinterpret_cast<f4*>(v) + i);
+      f4 wv = __builtin_nontemporal_load(reinterpret_cast<f4*>(w) + i);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        float a = mv[j], b = vv[j], c = wv[j];
+        step(gv[j], a, b, c);
+        mv[j] = a, vv[j] = b, wv[j] = c;
+      }
+      __builtin_nontemporal_store(mv, reinterpret_cast<f4*>(m) + i);
+      __builtin_nontemporal_store(vv, reinterpret_cast<f4*>(v) + i);
+      __builtin_nontemporal_store(wv, reinterpret_cast<f4*>(w) + i);
+    } else {
+      step(g[i], m[i], v[i], w[i]);
+    }
+  }
+  if (V > 1 && blockIdx.x == 0 && threadIdx.x < n % V) {
+    const size_t i = n - n % V + threadIdx.x;
+    step(g[i], m[i], v[i], w[i]);
   }
 }
 
@@ -1423,9 +1449,14 @@ int fh_op_adamw_step(fh_context* c, void* w, const void* g, void* m, void* v, in
   const float bc1 = 1.f - powf(beta1, (float)step);
   const float bc2 = 1.f - powf(beta2, (float)step);
   const int decay = weight_decay != 0.f && is_matrix;
-  hipLaunchKernelGGL(k_adamw, dim3(grid_for((size_t)n)), dim3(kT), 0, st_, static_cast<float*>(w),
-                     static_cast<const float*>(g), static_cast<float*>(m), static_cast<float*>(v), (size_t)n, lr,
-                     beta1, beta2, eps, weight_decay, bc1, bc2, decay);
+  float *fw = static_cast<float*>(w), *fm = static_cast<float*>(m), *fv = static_cast<float*>(v);
+  const float* fg = static_cast<const float*>(g);
+  if (aligned16(w) && aligned16(g) && aligned16(m) && aligned16(v))
+    hipLaunchKernelGGL(k_adamw<4>, dim3(grid_for(((size_t)n + 3) / 4)), dim3(kT), 0, st_, fw, fg, fm, fv, (size_t)n, lr,
+                       beta1, beta2, eps, weight_decay, bc1, bc2, decay);
+  else
+    hipLaunchKernelGGL(k_adamw<1>, dim3(grid_for((size_t)n)), dim3(kT), 0, st_, fw, fg, fm, fv, (size_t)n, lr, beta1,
+                       beta2, eps, weight_decay, bc1, bc2, decay);
   return op_launched("adamw step");
 }
 

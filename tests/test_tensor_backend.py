@@ -952,3 +952,27 @@ def test_unpack_qkv_zeroes_what_it_does_not_fill(fhp, tb, rows, cols):
     for i, t in enumerate(qkv):
         want[:B * T, 4 * i:4 * i + 4] = t.Data.reshape(B, H, T, hd).transpose(0, 2, 1, 3).reshape(B * T, 4)
     np.testing.assert_array_equal(dst.Data.reshape(rows, cols), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 100001])
+def test_adamw_lengths(fhp, tb, n):
+    """Lengths around the 16-byte groups: every element stepped once, against float64 (a few roundings)."""
+    g = np.random.default_rng(n)
+    w, gr, m = (g.standard_normal((3, n)) * 0.1).astype(np.float32)
+    v = (g.random(n) * 1e-2 + 1e-4).astype(np.float32)
+    t = [dup(fhp, a, 1, n) for a in (w, gr, m, v)]
+    tb.AdamWStep(*t, 1e-2, 0.9, 0.99, 1e-8, 0.1, 3)
+    for x in t:
+        tb.EnsureHostCurrent(x)
+    f = lambda x: float(np.float32(x))  # noqa: E731 - fp32 hyperparameters
+    b1, b2, lr, wd = f(0.9), f(0.99), f(1e-2), f(0.1)
+    m64 = b1 * m.astype(np.float64) + (1 - b1) * gr
+    v64 = b2 * v.astype(np.float64) + (1 - b2) * gr.astype(np.float64) ** 2
+    w64 = w.astype(np.float64) * (1 - lr * wd)
+    up = lr * (m64 / (1 - b1 ** 3)) / (np.sqrt(v64 / (1 - b2 ** 3)) + f(1e-8))
+    ulp = 2.0 ** -24
+    assert np.all(np.abs(t[2].Data - m64) <= 8 * ulp * (np.abs(m) + np.abs(gr)))
+    assert np.all(np.abs(t[3].Data - v64) <= 8 * ulp * (v + gr ** 2))
+    # the bias corrections 1 - b^3 lose up to 4 bits in fp32
+    assert np.all(np.abs(t[0].Data - (w64 - up)) <= 8 * ulp * np.abs(w) + 256 * ulp * (np.abs(up) + lr))
