@@ -176,6 +176,11 @@ struct Operand {
 template <int BM, int BN, bool AKC, bool BKC>
 __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 accumulators per wave (2 x 2 waves)
+  // The 64 x 64 tile has registers for a second accumulator: the five small products go there, so
+  // the large sums are rounded K / 16 times and not 6 K / 16 (48 heads of 331 x 64: 3.4e-7 -> 1.4e-7
+  // against 64 bits; windows of 33 to 128 rows at d 128: 2.6e-7 -> 1.8e-7, fp32 instructions 2.3e-7) at
+  // the same time.  128 x 64 would take 156 registers where it has 127: three blocks a CU, not four.
+  constexpr int NACC = MT * NT > 1 ? 1 : 2;
   __shared__ __align__(16) char smem[3 * (BM + BN) * 64];
   char* const As = smem;
   char* const Bs = smem + 3 * BM * 64;
@@ -205,13 +210,16 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   ob.init(b, BKC ? g.K : g.N, g.N, n0, g.K, kb, tid);
   float va[MT][8], vb[NT][8];
 
-  f32x16_t acc[MT][NT];
+  // acc[0]: the x1 y1 products, acc[1] (the same where registers are short) the five small ones
+  f32x16_t acc[NACC][MT][NT];
 #pragma unroll
-  for (int i = 0; i < MT; i++)
+  for (int c = 0; c < NACC; c++)
 #pragma unroll
-    for (int j = 0; j < NT; j++)
+    for (int i = 0; i < MT; i++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[c][i][j][r] = 0.f;
 
   auto compute = [&]() {
 #pragma unroll
@@ -236,7 +244,8 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
         for (int i = 0; i < MT; i++)
 #pragma unroll
           for (int j = 0; j < NT; j++)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[PA[p]][i], bf[PB[p]][j], acc[i][j], 0, 0, 0);
+            acc[p < 5 ? NACC - 1 : 0][i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                af[PA[p]][i], bf[PB[p]][j], acc[p < 5 ? NACC - 1 : 0][i][j], 0, 0, 0);
     }
   };
 
@@ -245,11 +254,13 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   auto flip = [&]() {
     sign ^= 0x80000000u;
 #pragma unroll
-    for (int i = 0; i < MT; i++)
+    for (int c = 0; c < NACC; c++)
 #pragma unroll
-      for (int j = 0; j < NT; j++)
+      for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[i][j][r] = -acc[i][j][r];
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) acc[c][i][j][r] = -acc[c][i][j][r];
   };
   auto put = [&]() {
     oa.store(As, va, sign);
@@ -280,6 +291,14 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
     compute();
   }
   if (sign) flip();
+  if constexpr (NACC == 2) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[0][i][j][r] += acc[1][i][j][r];
+  }
 
   // ---- results ------------------------------------------------------------------------
   const size_t yrow = (size_t)slot * g.M + m0;
@@ -294,7 +313,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
       const bool in_n = n0 + wn * (BN / 2) + j * 32 + fr < g.N;
 #pragma unroll
       for (int r = 0; r < 16; r++)
-        bad |= in_n && wm * (BM / 2) + i * 32 + mfma_acc_row(lane, r) < rows && !(fabsf(acc[i][j][r]) < INFINITY);
+        bad |= in_n && wm * (BM / 2) + i * 32 + mfma_acc_row(lane, r) < rows && !(fabsf(acc[0][i][j][r]) < INFINITY);
     }
   if (__syncthreads_or(bad)) {
     // not all finite: the tile by fp32 multiply-adds in k order
@@ -326,13 +345,13 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
     for (int i = 0; i < MT; i++) {
       const int tr = wm * (BM / 2) + i * 32;
       if (parts)
-        mfma_store_tile<EPI_NONE, false, false, 2>(acc[i][j], lane, tr, col, g.N, 0.f, ry, ry);
+        mfma_store_tile<EPI_NONE, false, false, 2>(acc[0][i][j], lane, tr, col, g.N, 0.f, ry, ry);
       else if (g.gelu)
-        mfma_store_tile<EPI_GELU, false, false>(acc[i][j], lane, tr, col, g.N, bcol, ry, ry);
+        mfma_store_tile<EPI_GELU, false, false>(acc[0][i][j], lane, tr, col, g.N, bcol, ry, ry);
       else if (g.res)
-        mfma_store_tile<EPI_NONE, true, false>(acc[i][j], lane, tr, col, g.N, bcol, rres, ry);
+        mfma_store_tile<EPI_NONE, true, false>(acc[0][i][j], lane, tr, col, g.N, bcol, rres, ry);
       else
-        mfma_store_tile<EPI_NONE, false, false>(acc[i][j], lane, tr, col, g.N, bcol, ry, ry);
+        mfma_store_tile<EPI_NONE, false, false>(acc[0][i][j], lane, tr, col, g.N, bcol, ry, ry);
     }
   }
 }
