@@ -145,28 +145,34 @@ __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, con
 // HBM-bound copies.  A block row (blockIdx.y) is one (sequence, head) slot, so a thread
 // divides by the head's width alone, and V (4 where widths, offsets and pointers are
 // multiples of 16 bytes) floats move per load (48 slots of 331 x 64: 5.9 -> 3.4 us; three
-// divisions per float before).
+// divisions per float before).  blockIdx.z is one of up to three packed tensors whose columns
+// follow each other (q, k and v in one launch: 4.9 us for three of 4 MB, 3.4 for one).
+struct PackSlices {
+  float* packed[3];
+};
 template <int V>
-__global__ __launch_bounds__(256) void k_pack_heads(const float* __restrict__ src, int src_cols,
-                                                    float* __restrict__ dst, int slots, int T, int H, int hd,
-                                                    int col_base, int unpack) {
+__global__ __launch_bounds__(256) void k_pack_heads(float* __restrict__ wide, int wide_cols, PackSlices slices,
+                                                    int slots, int T, int H, int hd, int col_base, int unpack) {
   const unsigned per = hd / V, n = (unsigned)T * per;
+  float* __restrict__ const packed = slices.packed[blockIdx.z];
+  const int col = col_base + blockIdx.z * H * hd;
   for (int s = blockIdx.y; s < slots; s += gridDim.y) {
     const int q = s / H, h = s % H;
-    const size_t wide0 = (size_t)q * T * src_cols + col_base + h * hd, packed0 = (size_t)s * T * hd;
+    const size_t wide0 = (size_t)q * T * wide_cols + col + h * hd, packed0 = (size_t)s * T * hd;
     for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
       const unsigned t = i / per, e = i % per * V;
-      const size_t wide = wide0 + (size_t)t * src_cols + e, packed = packed0 + (size_t)i * V;
+      float* const pw = wide + wide0 + (size_t)t * wide_cols + e;
+      float* const pp = packed + packed0 + (size_t)i * V;
       if constexpr (V == 4) {
         if (unpack)
-          *reinterpret_cast<float4*>(dst + wide) = *reinterpret_cast<const float4*>(src + packed);
+          *reinterpret_cast<float4*>(pw) = *reinterpret_cast<const float4*>(pp);
         else
-          *reinterpret_cast<float4*>(dst + packed) = *reinterpret_cast<const float4*>(src + wide);
+          *reinterpret_cast<float4*>(pp) = *reinterpret_cast<const float4*>(pw);
       } else {
         if (unpack)
-          dst[wide] = src[packed];
+          *pw = *pp;
         else
-          dst[packed] = src[wide];
+          *pp = *pw;
       }
     }
   }
@@ -1029,16 +1035,18 @@ int matmul_common(fh_context* c, int mode, const void* a, const void* b, void* y
   return op_launched("matmul");
 }
 
-void launch_pack(hipStream_t st, const float* src, int wide_cols, float* dst, int batch, int T, int H, int hd,
-                 int col_base, int unpack) {
-  const bool v4 = hd % 4 == 0 && wide_cols % 4 == 0 && col_base % 4 == 0 && aligned16(src) && aligned16(dst);
+// `count` packed tensors of slots * T * hd floats each, from (unpack: into) columns that follow each
+// other in the wide rows
+int launch_pack(hipStream_t st, float* wide, int wide_cols, const PackSlices& p, int count, int batch, int T, int H,
+                int hd, int col_base, int unpack) {
+  bool v4 = hd % 4 == 0 && wide_cols % 4 == 0 && col_base % 4 == 0 && aligned16(wide);
+  for (int i = 0; i < count; i++) v4 = v4 && aligned16(p.packed[i]);
   const size_t n = (size_t)T * hd / (v4 ? 4 : 1);
   const int slots = batch * H;
-  const dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 65535), (unsigned)std::min(slots, 65535));
-  if (v4)
-    hipLaunchKernelGGL(k_pack_heads<4>, grid, dim3(256), 0, st, src, wide_cols, dst, slots, T, H, hd, col_base, unpack);
-  else
-    hipLaunchKernelGGL(k_pack_heads<1>, grid, dim3(256), 0, st, src, wide_cols, dst, slots, T, H, hd, col_base, unpack);
+  const dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 65535), (unsigned)std::min(slots, 65535), count);
+  hipLaunchKernelGGL(v4 ? k_pack_heads<4> : k_pack_heads<1>, grid, dim3(256), 0, st, wide, wide_cols, p, slots, T, H, hd,
+                     col_base, unpack);
+  return op_launched(unpack ? "unpack heads" : "pack heads");
 }
 
 int softmax_common(fh_context* c, void* x, int rows, int cols, float scale, int causal) {
@@ -1074,9 +1082,8 @@ int fh_op_pack_heads(fh_context* c, const void* src, int src_cols, void* dst, in
   OPS_ARG(batch > 0 && T > 0 && n_heads > 0 && head_dim > 0 && col_base >= 0 &&
               col_base + n_heads * head_dim <= src_cols,
           "head slices outside the source rows");
-  launch_pack(st_, static_cast<const float*>(src), src_cols, static_cast<float*>(dst), batch, T, n_heads, head_dim,
-              col_base, 0);
-  return op_launched("pack heads");
+  return launch_pack(st_, static_cast<float*>(const_cast<void*>(src)), src_cols, PackSlices{{static_cast<float*>(dst)}},
+                     1, batch, T, n_heads, head_dim, col_base, 0);
 }
 
 int fh_op_unpack_heads(fh_context* c, const void* src, void* dst, int dst_cols, int batch, int T, int n_heads,
@@ -1086,9 +1093,31 @@ int fh_op_unpack_heads(fh_context* c, const void* src, void* dst, int dst_cols, 
   OPS_ARG(batch > 0 && T > 0 && n_heads > 0 && head_dim > 0 && col_base >= 0 &&
               col_base + n_heads * head_dim <= dst_cols,
           "head slices outside the destination rows");
-  launch_pack(st_, static_cast<const float*>(src), dst_cols, static_cast<float*>(dst), batch, T, n_heads, head_dim,
-              col_base, 1);
-  return op_launched("unpack heads");
+  return launch_pack(st_, static_cast<float*>(dst), dst_cols,
+                     PackSlices{{static_cast<float*>(const_cast<void*>(src))}}, 1, batch, T, n_heads, head_dim,
+                     col_base, 1);
+}
+
+int fh_op_pack_qkv_heads(fh_context* c, const void* src, int src_cols, void* q, void* k, void* v, int batch, int T,
+                         int n_heads, int head_dim) {
+  OPS_PROLOGUE(c);
+  OPS_ARG(src && q && k && v, "null buffer");
+  OPS_ARG(batch > 0 && T > 0 && n_heads > 0 && head_dim > 0 && 3ll * n_heads * head_dim <= src_cols,
+          "head slices outside the source rows");
+  return launch_pack(st_, static_cast<float*>(const_cast<void*>(src)), src_cols,
+                     PackSlices{{static_cast<float*>(q), static_cast<float*>(k), static_cast<float*>(v)}}, 3, batch, T,
+                     n_heads, head_dim, 0, 0);
+}
+
+int fh_op_unpack_qkv_heads(fh_context* c, const void* q, const void* k, const void* v, void* dst, int dst_cols,
+                           int batch, int T, int n_heads, int head_dim) {
+  OPS_PROLOGUE(c);
+  OPS_ARG(q && k && v && dst, "null buffer");
+  OPS_ARG(batch > 0 && T > 0 && n_heads > 0 && head_dim > 0 && 3ll * n_heads * head_dim <= dst_cols,
+          "head slices outside the destination rows");
+  auto f = [](const void* p) { return static_cast<float*>(const_cast<void*>(p)); };
+  return launch_pack(st_, static_cast<float*>(dst), dst_cols, PackSlices{{f(q), f(k), f(v)}}, 3, batch, T, n_heads,
+                     head_dim, 0, 1);
 }
 
 int fh_op_add_bias(fh_context* c, void* y, const void* bias, int rows, int cols) {

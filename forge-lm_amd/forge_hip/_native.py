@@ -38,6 +38,7 @@ EXPORTS = (
     "fh_checkpoint_info", "fh_session_load_checkpoint", "fh_sha256", "fh_generate_begin", "fh_generate_next",
     # op-level ITensorBackend
     "fh_op_matmul_nn", "fh_op_matmul_nt", "fh_op_matmul_tn", "fh_op_pack_heads", "fh_op_unpack_heads",
+    "fh_op_pack_qkv_heads", "fh_op_unpack_qkv_heads",
     "fh_op_add_bias", "fh_op_sum_rows", "fh_op_add_in_place", "fh_op_copy", "fh_op_scale", "fh_op_zero",
     "fh_op_copy_block", "fh_op_transpose", "fh_op_layernorm_forward", "fh_op_layernorm_backward",
     "fh_op_softmax_forward", "fh_op_scaled_causal_softmax_forward", "fh_op_softmax_backward",
@@ -134,6 +135,8 @@ def lib():
         getattr(L, f"fh_op_matmul_{mm}").argtypes = [vp, vp, vp, vp, ci, ci, ci, ci, ci]
     L.fh_op_pack_heads.argtypes = [vp, vp, ci, vp, ci, ci, ci, ci, ci]
     L.fh_op_unpack_heads.argtypes = [vp, vp, vp, ci, ci, ci, ci, ci, ci]
+    L.fh_op_pack_qkv_heads.argtypes = [vp, vp, ci, vp, vp, vp, ci, ci, ci, ci]
+    L.fh_op_unpack_qkv_heads.argtypes = [vp, vp, vp, vp, vp, ci, ci, ci, ci, ci]
     L.fh_op_add_bias.argtypes = [vp, vp, vp, ci, ci]
     L.fh_op_sum_rows.argtypes = [vp, vp, vp, ci, ci]
     L.fh_op_add_in_place.argtypes = [vp, vp, vp, i64]

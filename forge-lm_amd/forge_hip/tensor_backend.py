@@ -194,6 +194,11 @@ class HipTensorBackend:
     def PackQkvHeads(self, src, q, k, v, batch, T, nHeads, headDim):
         """ITensorBackend.cs:58-65."""
         d = nHeads * headDim
+        if min(batch, T, nHeads, headDim) > 0 and 3 * d <= src.Cols and len({id(t) for t in (src, q, k, v)}) == 4:
+            ps = self._read(src)
+            N.check(N.lib().fh_op_pack_qkv_heads(self._ctx, ps, src.Cols, self._write(q), self._write(k),
+                                                 self._write(v), batch, T, nHeads, headDim))
+            return
         self.PackHeads(src, q, batch, T, nHeads, headDim, 0)
         self.PackHeads(src, k, batch, T, nHeads, headDim, d)
         self.PackHeads(src, v, batch, T, nHeads, headDim, 2 * d)
@@ -205,6 +210,11 @@ class HipTensorBackend:
             self._write(dst)  # the three slices fill it: no zeros to write, no host copy to upload
         else:
             self.Zero(dst)
+        if min(batch, T, nHeads, headDim) > 0 and 3 * d <= dst.Cols and not any(t is dst for t in (q, k, v)):
+            pq, pk, pv = self._read(q), self._read(k), self._read(v)
+            N.check(N.lib().fh_op_unpack_qkv_heads(self._ctx, pq, pk, pv, self._write(dst, preserve=True), dst.Cols,
+                                                   batch, T, nHeads, headDim))
+            return
         self.UnpackHeads(q, dst, batch, T, nHeads, headDim, 0)
         self.UnpackHeads(k, dst, batch, T, nHeads, headDim, d)
         self.UnpackHeads(v, dst, batch, T, nHeads, headDim, 2 * d)

@@ -264,6 +264,12 @@ int fh_op_pack_heads(fh_context* ctx, const void* src, int src_cols, void* dst, 
                      int head_dim, int col_base);
 int fh_op_unpack_heads(fh_context* ctx, const void* src, void* dst, int dst_cols, int batch, int T, int n_heads,
                        int head_dim, int col_base);
+/* PackQkvHeads (:58-65): q, k and v (distinct buffers) from columns 0, n_heads * head_dim and twice that,
+ * in one launch; UnpackQkvHeads (:68-76) back, other columns of dst left as they are. */
+int fh_op_pack_qkv_heads(fh_context* ctx, const void* src, int src_cols, void* q, void* k, void* v, int batch, int T,
+                         int n_heads, int head_dim);
+int fh_op_unpack_qkv_heads(fh_context* ctx, const void* q, const void* k, const void* v, void* dst, int dst_cols,
+                           int batch, int T, int n_heads, int head_dim);
 /* AddBias (:80) y[r,:] += bias; SumRows (:82) dbias += column sums of dy (accumulates). */
 int fh_op_add_bias(fh_context* ctx, void* y, const void* bias, int rows, int cols);
 int fh_op_sum_rows(fh_context* ctx, const void* dy, void* dbias, int rows, int cols);

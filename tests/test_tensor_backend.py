@@ -976,3 +976,29 @@ def test_adamw_lengths(fhp, tb, n):
     assert np.all(np.abs(t[3].Data - v64) <= 8 * ulp * (v + gr ** 2))
     # the bias corrections 1 - b^3 lose up to 4 bits in fp32
     assert np.all(np.abs(t[0].Data - (w64 - up)) <= 8 * ulp * np.abs(w) + 256 * ulp * (np.abs(up) + lr))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,extra", [(8, 0), (8, 4), (8, 3), (6, 0)])
+def test_pack_qkv_in_one_launch(fhp, tb, hd, extra):
+    """Widths by 16 bytes and not, rows wider than the three slices, and one tensor for two of them
+    (the later slice stays, as in three packs)."""
+    g = np.random.default_rng(hd + extra)
+    B, T, H = 2, 37, 3
+    d = H * hd
+    src = g.standard_normal((B * T, 3 * d + extra)).astype(np.float32)
+    want = [src[:, i * d:(i + 1) * d].reshape(B, T, H, hd).transpose(0, 2, 1, 3).reshape(-1, hd) for i in range(3)]
+    ts = dup(fhp, src, B * T, 3 * d + extra)
+    q, k, v = (fhp.Tensor(B * H * T, hd) for _ in range(3))
+    tb.PackQkvHeads(ts, q, k, v, B, T, H, hd)
+    for t, w in zip((q, k, v), want):
+        tb.EnsureHostCurrent(t)
+        np.testing.assert_array_equal(t.Data.reshape(w.shape), w)
+    back = fhp.Tensor(B * T, 3 * d + extra)
+    tb.UnpackQkvHeads(q, k, v, back, B, T, H, hd)
+    tb.EnsureHostCurrent(back)
+    np.testing.assert_array_equal(back.Data.reshape(src.shape)[:, :3 * d], src[:, :3 * d])
+    assert np.all(back.Data.reshape(src.shape)[:, 3 * d:] == 0)
+    tb.PackQkvHeads(ts, q, q, v, B, T, H, hd)
+    tb.EnsureHostCurrent(q)
+    np.testing.assert_array_equal(q.Data.reshape(want[1].shape), want[1])
