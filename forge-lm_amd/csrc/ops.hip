@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -76,6 +77,7 @@ __device__ __forceinline__ double block_sum_double(double s, double* red) {
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 unsigned grid_for(size_t n) { return (unsigned)std::min<size_t>((n + kT - 1) / kT, 65536); }
+unsigned grid_vec(size_t n, bool v4) { return grid_for(v4 ? (n + 3) / 4 : n); }
 
 // ---- matmuls: y[s] (+)= op(a[s]) @ op(b[s]), 64x64 tiles, k steps of 16 ------------
 // for sizes that the split GEMM does not take (gemm_split_fits), with 64-bit offsets
@@ -179,15 +181,63 @@ __global__ __launch_bounds__(256) void k_pack_heads(float* __restrict__ wide, in
 }
 
 // ---- elementwise and row kernels -----------------------------------------------------
-__global__ void k_add_bias(float* __restrict__ y, const float* __restrict__ bias, int rows, int cols) {
-  const size_t n = (size_t)rows * cols;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    y[i] = y[i] + bias[i % cols];
+// Elementwise kernels: V floats (4 where the pointers, and for a bias its rows, are multiples of 16
+// bytes) to a load, the last n % V by the first block's threads.
+template <int V, typename F>
+__device__ __forceinline__ void each_vec(size_t n, F f) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n / V; i += (size_t)gridDim.x * 256)
+    f(i * V, std::integral_constant<int, V>());
+  if (V > 1 && blockIdx.x == 0 && threadIdx.x < n % V) f(n - n % V + threadIdx.x, std::integral_constant<int, 1>());
 }
 
-__global__ void k_add_in_place(float* __restrict__ dst, const float* __restrict__ src, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    dst[i] = dst[i] + src[i];
+template <int V>
+struct Floats {
+  float v[V];
+  __device__ __forceinline__ void load(const float* p) {
+    if constexpr (V == 4) {
+      const float4 t = *reinterpret_cast<const float4*>(p);
+      v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
+    } else {
+      v[0] = *p;
+    }
+  }
+  __device__ __forceinline__ void store(float* p) const {
+    if constexpr (V == 4)
+      *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+      *p = v[0];
+  }
+};
+
+// HBM-bound: a block row (blockIdx.y) takes every gridDim.y-th row, so no element divides by the row's
+// width (2048 x 3072: 14.6 -> 8.8 us)
+template <int V>
+__global__ __launch_bounds__(256) void k_add_bias(float* __restrict__ y, const float* __restrict__ bias, int rows,
+                                                  int cols) {
+  const unsigned c = (blockIdx.x * 256 + threadIdx.x) * V;
+  if (c >= (unsigned)cols) return;
+  Floats<V> b, t;
+  b.load(bias + c);
+#pragma unroll 4
+  for (int r = blockIdx.y; r < rows; r += gridDim.y) {
+    float* const p = y + (size_t)r * cols + c;
+    t.load(p);
+#pragma unroll
+    for (int j = 0; j < V; j++) t.v[j] = t.v[j] + b.v[j];
+    t.store(p);
+  }
+}
+
+template <int V>
+__global__ __launch_bounds__(256) void k_add_in_place(float* dst, const float* src, size_t n) {
+  each_vec<V>(n, [&](size_t i, auto w) {
+    Floats<decltype(w)::value> a, b;
+    a.load(dst + i);
+    b.load(src + i);
+#pragma unroll
+    for (int j = 0; j < decltype(w)::value; j++) a.v[j] = a.v[j] + b.v[j];
+    a.store(dst + i);
+  });
 }
 
 __global__ void k_scale(float* __restrict__ x, size_t n, float f) {
@@ -552,20 +602,38 @@ constexpr int kRowWaveCols = 1024;
 // ---- GELU (CpuBackend.cs:477-514) ------------------------------------------------------
 __device__ __forceinline__ float gelu_c() { return 0.7978845238685608f; }  // MathF.Sqrt(2f / MathF.PI)
 
-__global__ void k_gelu_forward(const float* __restrict__ x, float* __restrict__ out, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    out[i] = gelu_tanh(x[i]);
+// (1 + tanh u) / 2 is 1 / (1 + e^-2u): one exponential and a division where tanhf took both of its
+// branches, and no cancellation where tanh u is near -1.  tanhf bound both kernels on the VALU; with 16
+// bytes to a load they are HBM-bound (2048 x 3072: forward 13.3 -> 9.3 us, backward 18.8 -> 12.4).
+__device__ __forceinline__ float gelu_gate(float v) {
+  return 1.f / (1.f + expf(-2.f * (gelu_c() * (v + 0.044715f * v * v * v))));
 }
 
-__global__ void k_gelu_backward(const float* __restrict__ dout, const float* __restrict__ x, float* __restrict__ dx,
-                                size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const float v = x[i];
-    const float u = gelu_c() * (v + 0.044715f * v * v * v);
-    const float t = tanhf(u);
-    const float du = gelu_c() * (1.f + 3.f * 0.044715f * v * v);
-    dx[i] = dout[i] * 0.5f * (1.f + t + v * (1.f - t * t) * du);
-  }
+template <int V>
+__global__ __launch_bounds__(256) void k_gelu_forward(const float* x, float* out, size_t n) {
+  each_vec<V>(n, [&](size_t i, auto w) {
+    Floats<decltype(w)::value> a;
+    a.load(x + i);
+#pragma unroll
+    for (int j = 0; j < decltype(w)::value; j++) a.v[j] = a.v[j] * gelu_gate(a.v[j]);
+    a.store(out + i);
+  });
+}
+
+template <int V>
+__global__ __launch_bounds__(256) void k_gelu_backward(const float* dout, const float* x, float* dx, size_t n) {
+  each_vec<V>(n, [&](size_t i, auto w) {
+    Floats<decltype(w)::value> a, d;
+    a.load(x + i);
+    d.load(dout + i);
+#pragma unroll
+    for (int j = 0; j < decltype(w)::value; j++) {
+      const float v = a.v[j], g = gelu_gate(v);
+      const float du = gelu_c() * (1.f + 3.f * 0.044715f * v * v);
+      d.v[j] = d.v[j] * (g + v * (2.f * g * (1.f - g)) * du);
+    }
+    d.store(dx + i);
+  });
 }
 
 // ---- embedding (CpuBackend.cs:518-543) ----------------------------------------------------
@@ -1123,8 +1191,11 @@ int fh_op_unpack_qkv_heads(fh_context* c, const void* q, const void* k, const vo
 int fh_op_add_bias(fh_context* c, void* y, const void* bias, int rows, int cols) {
   OPS_PROLOGUE(c);
   OPS_ARG(y && bias && rows > 0 && cols > 0, "bad arguments");
-  const size_t n = (size_t)rows * cols;
-  hipLaunchKernelGGL(k_add_bias, dim3(grid_for(n)), dim3(kT), 0, st_, static_cast<float*>(y),
+  const bool v4 = cols % 4 == 0 && aligned16(y) && aligned16(bias);
+  const int strips = (cols / (v4 ? 4 : 1) + 255) / 256;
+  // about 4096 blocks, so that a long column has several rows to a thread
+  const dim3 grid(strips, std::max(1, std::min({rows, (4096 + strips - 1) / strips, 65535})));
+  hipLaunchKernelGGL(v4 ? k_add_bias<4> : k_add_bias<1>, grid, dim3(256), 0, st_, static_cast<float*>(y),
                      static_cast<const float*>(bias), rows, cols);
   return op_launched("add bias");
 }
@@ -1154,7 +1225,9 @@ int fh_op_sum_rows(fh_context* c, const void* dy, void* dbias, int rows, int col
 int fh_op_add_in_place(fh_context* c, void* dst, const void* src, int64_t n) {
   OPS_PROLOGUE(c);
   OPS_ARG(dst && src && n > 0, "bad arguments");
-  hipLaunchKernelGGL(k_add_in_place, dim3(grid_for((size_t)n)), dim3(kT), 0, st_, static_cast<float*>(dst),
+  const bool v4 = aligned16(dst) && aligned16(src);
+  hipLaunchKernelGGL(v4 ? k_add_in_place<4> : k_add_in_place<1>, dim3(grid_vec((size_t)n, v4)), dim3(256), 0, st_,
+                     static_cast<float*>(dst),
                      static_cast<const float*>(src), (size_t)n);
   return op_launched("add in place");
 }
@@ -1258,7 +1331,9 @@ int fh_op_softmax_backward(fh_context* c, const void* dout, const void* sm, void
 int fh_op_gelu_forward(fh_context* c, const void* x, void* out, int64_t n) {
   OPS_PROLOGUE(c);
   OPS_ARG(x && out && n > 0, "bad arguments");
-  hipLaunchKernelGGL(k_gelu_forward, dim3(grid_for((size_t)n)), dim3(kT), 0, st_, static_cast<const float*>(x),
+  const bool v4 = aligned16(x) && aligned16(out);
+  hipLaunchKernelGGL(v4 ? k_gelu_forward<4> : k_gelu_forward<1>, dim3(grid_vec((size_t)n, v4)), dim3(256), 0, st_,
+                     static_cast<const float*>(x),
                      static_cast<float*>(out), (size_t)n);
   return op_launched("gelu forward");
 }
@@ -1266,7 +1341,9 @@ int fh_op_gelu_forward(fh_context* c, const void* x, void* out, int64_t n) {
 int fh_op_gelu_backward(fh_context* c, const void* dout, const void* x, void* dx, int64_t n) {
   OPS_PROLOGUE(c);
   OPS_ARG(dout && x && dx && n > 0, "bad arguments");
-  hipLaunchKernelGGL(k_gelu_backward, dim3(grid_for((size_t)n)), dim3(kT), 0, st_, static_cast<const float*>(dout),
+  const bool v4 = aligned16(dout) && aligned16(x) && aligned16(dx);
+  hipLaunchKernelGGL(v4 ? k_gelu_backward<4> : k_gelu_backward<1>, dim3(grid_vec((size_t)n, v4)), dim3(256), 0, st_,
+                     static_cast<const float*>(dout),
                      static_cast<const float*>(x), static_cast<float*>(dx), (size_t)n);
   return op_launched("gelu backward");
 }

@@ -978,6 +978,71 @@ def test_adamw_lengths(fhp, tb, n):
     assert np.all(np.abs(t[0].Data - (w64 - up)) <= 8 * ulp * np.abs(w) + 256 * ulp * (np.abs(up) + lr))
 
 
+def _gelu64(x):
+    """GELU (tanh form) and its derivative in float64; 1 + tanh u as 2 / (1 + e^-2u), which keeps the tail."""
+    x = x.astype(np.float64)
+    c = np.sqrt(2 / np.pi)
+    g = 1 / (1 + np.exp(-2 * c * (x + 0.044715 * x ** 3)))
+    return x * g, g + 2 * x * g * (1 - g) * c * (1 + 3 * 0.044715 * x * x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1028, 300001])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_elementwise_lengths_and_alignment(fhp, tb, n, offset):
+    """Lengths around the 16-byte groups, pointers on and off 16 bytes: every element once, none past the end.
+
+    GELU's gate is 1 / (1 + e^-2u): a relative error of e^-2u is that of 2u (4 roundings of up to 2|u| < 14 for
+    |x| < 4) and a few ulp of exp, add and divide."""
+    import ctypes
+    from forge_hip import _native as N
+    g = np.random.default_rng(n)
+    x, d = np.clip(g.standard_normal((2, n + 2)), -4, 4).astype(np.float32)
+    t = {k: dup(fhp, a, 1, n + 2) for k, a in dict(x=x, d=d, f=x * 0 + 7, b=x * 0 + 7, a=x).items()}
+    at = {k: ctypes.c_void_p(tb._write(v, preserve=True).value + 4 * offset) for k, v in t.items()}
+    L, ctx = N.lib(), tb._ctx
+    N.check(L.fh_op_gelu_forward(ctx, at["x"], at["f"], n))
+    N.check(L.fh_op_gelu_backward(ctx, at["d"], at["x"], at["b"], n))
+    N.check(L.fh_op_add_in_place(ctx, at["a"], at["d"], n))
+    for v in t.values():
+        tb.EnsureHostCurrent(v)
+    s = slice(offset, offset + n)
+    f64, b64 = _gelu64(x[s])
+    ulp = 2.0 ** -24
+    assert np.all(np.abs(t["f"].Data[s] - f64) <= 80 * ulp * np.abs(f64) + 1e-30)
+    # the derivative's terms reach 1.2 each and cancel
+    assert np.all(np.abs(t["b"].Data[s] - d[s] * b64) <= 80 * ulp * np.abs(d[s]) * 1.2 + 1e-30)
+    np.testing.assert_array_equal(t["a"].Data[s], x[s] + d[s])
+    rest = np.r_[0:offset, offset + n:n + 2]
+    assert np.all(t["f"].Data[rest] == 7) and np.all(t["b"].Data[rest] == 7)
+    np.testing.assert_array_equal(t["a"].Data[rest], x[rest])
+
+
+@pytest.mark.gpu
+def test_gelu_of_infinities_and_nan(fhp, oracle, tb):
+    """What 0.5 x (1 + tanh u) gives: NaN at -inf and NaN, inf at inf, signed zeros of the tails."""
+    x = np.array([-np.inf, np.inf, np.nan, -100, 100, -1e15, 1e15, 0.0, -0.0], np.float32)
+    xt, out, dx = dup(fhp, x, 1, 9), fhp.Tensor(1, 9), fhp.Tensor(1, 9)
+    tb.GeluForward(xt, out)
+    tb.GeluBackward(dup(fhp, np.ones(9, np.float32), 1, 9), xt, dx)
+    tb.EnsureHostCurrent(out)
+    tb.EnsureHostCurrent(dx)
+    np.testing.assert_array_equal(out.Data, np.array([np.nan, np.inf, np.nan, 0, 100, 0, 1e15, 0, 0], np.float32))
+    np.testing.assert_array_equal(dx.Data, np.array([np.nan, np.nan, np.nan, 0, 1, 0, 1, 0.5, 0.5], np.float32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4), (5, 1023), (2, 1028), (9000, 8)])
+def test_add_bias_shapes(fhp, tb, rows, cols):
+    """Rows by 16 bytes and by 4, a last strip in part, more rows than block rows: one addition each."""
+    g = np.random.default_rng(rows + cols)
+    y, b = g.standard_normal((rows, cols)).astype(np.float32), g.standard_normal(cols).astype(np.float32)
+    t = dup(fhp, y, rows, cols)
+    tb.AddBias(t, dup(fhp, b, cols), rows, cols)
+    tb.EnsureHostCurrent(t)
+    np.testing.assert_array_equal(t.Data.reshape(rows, cols), y + b)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("hd,extra", [(8, 0), (8, 4), (8, 3), (6, 0)])
 def test_pack_qkv_in_one_launch(fhp, tb, hd, extra):
