@@ -161,6 +161,9 @@ __global__ __launch_bounds__(256) void k_layernorm_rows_bf16(const float* __rest
 // LayerNorm that follows: one 1024-thread block per row (a thread per column)
 // writes the row to y, exactly as k_splitk_epilogue would, and its LayerNorm to
 // out, with k_layernorm's formula over block sums.  N <= 1024.
+// U: partials asked for at once.  The smallest of 8, 16, 24 and 32 that holds S: a skipped load costs its
+// issue all the same (16 waves x 32 of them; with 8 the forward of 333 rows takes 1250 us, with 32 always 1272).
+template <int U>
 __global__ __launch_bounds__(1024) void k_epilogue_ln(const float* __restrict__ part, int S, int M, int N,
                                                       const float* __restrict__ bias, const float* __restrict__ res,
                                                       float* __restrict__ y, const float* __restrict__ w,
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(1024) void k_epilogue_ln(const float* __restrict__ 
   __shared__ float red[16];
   const int r = blockIdx.x, c = threadIdx.x;
   const bool on = c < N;
-  // one column per thread, up to 32 of its partials in flight together through a
+  // one column per thread, up to U of its partials in flight together through a
   // bounded resource (skipped ones, past S or N, read as zeros); the partials add
   // in order, and the zeros after the last one change nothing.  Each partial is
   // read once: the loads carry the non-temporal hint (C4: 870 -> 863 us per step).
@@ -188,15 +191,15 @@ __global__ __launch_bounds__(1024) void k_epilogue_ln(const float* __restrict__ 
     lbc = b[c];
   }
   float v = 0.f;
-  for (int i0 = 0; i0 < S; i0 += 32) {
-    float t[32];
+  for (int i0 = 0; i0 < S; i0 += U) {
+    float t[U];
 #pragma unroll
-    for (int ii = 0; ii < 32; ii++) {
+    for (int ii = 0; ii < U; ii++) {
       const int off = (on && i0 + ii < S) ? (int)((((size_t)(i0 + ii) * M + r) * N + c) * 4) : pbytes;
       t[ii] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rp, off, 0, 2));
     }
 #pragma unroll
-    for (int ii = 0; ii < 32; ii++) v += t[ii];
+    for (int ii = 0; ii < U; ii++) v += t[ii];
   }
   if (on) {
     if (bias) v += bc;
@@ -219,10 +222,10 @@ __global__ __launch_bounds__(256) void k_epilogue_qkv(const float* __restrict__ 
                                                       const float* __restrict__ bias, float* __restrict__ qkv,
                                                       RowSrc src, int T, int H, int ctx, KT* __restrict__ kc,
                                                       KT* __restrict__ vc) {
-  const int N = 3 * d;
+  const unsigned N = 3 * d;
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)M * N) return;
-  const int col = (int)(idx % N), r = (int)(idx / N);
+  const int r = (int)((unsigned)idx / N), col = (int)((unsigned)idx - r * N);  // M N < 2^32 (the launch checks)
   // the bias and the step counter are requested with the partials (a load issued
   // after the store of qkv would wait for it)
   const float bc = bias ? bias[col] : 0.f;
@@ -1517,7 +1520,11 @@ hipError_t launch_epilogue_ln(hipStream_t st, const float* part, int splits, int
                               const float* res, float* y, const float* w, const float* b, float* out, float eps) {
   FH_CHECK_ARG(splits >= 1 && M > 0 && N > 0 && N <= 1024 && part && y && w && b && out &&
                (size_t)splits * M * N * 4 < 0x7fffffffu);
-  hipLaunchKernelGGL(k_epilogue_ln, dim3(M), dim3(1024), 0, st, part, splits, M, N, bias, res, y, w, b, out, eps);
+  const auto kernel = splits <= 8    ? k_epilogue_ln<8>
+                      : splits <= 16 ? k_epilogue_ln<16>
+                      : splits <= 24 ? k_epilogue_ln<24>
+                                     : k_epilogue_ln<32>;
+  hipLaunchKernelGGL(kernel, dim3(M), dim3(1024), 0, st, part, splits, M, N, bias, res, y, w, b, out, eps);
   return hipGetLastError();
 }
 
@@ -1527,6 +1534,7 @@ hipError_t launch_epilogue_qkv(hipStream_t st, const float* part, int splits, in
   FH_CHECK_ARG(splits >= 1 && M > 0 && d > 0 && H > 0 && d % H == 0 && T > 0 && M % T == 0 && ctx > 0 && part &&
                qkv && kcache && vcache && src.step);
   const size_t tot = (size_t)M * 3 * d;
+  FH_CHECK_ARG(tot < 0x100000000ull);
   hipLaunchKernelGGL(k_epilogue_qkv<KT>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, part, splits, M, d,
                      bias, qkv, src, T, H, ctx, kcache, vcache);
   return hipGetLastError();

@@ -1231,3 +1231,17 @@ def test_fp32_window_attention_blocks_match_oracle(fhp, oracle, backend, B, T):
     for b in sorted({0, B // 2, B - 1}):
         _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
         assert rel_err(got[b], rlg[0]) <= TOL_F32
+
+
+@pytest.mark.parametrize("D,H", [(128, 4), (256, 4), (512, 8), (768, 12)])
+def test_fused_epilogue_split_counts_match_oracle(fhp, oracle, backend, D, H):
+    """The reductions with a LayerNorm at split counts over their groups of 8, 16, 24 and 32 partials: a
+    decode of 5 rows (attn.proj D / 32 splits, mlp.proj 32 and less) after windows of 40 and 190 rows in all."""
+    m, oc, w = make_model(fhp, oracle, backend, (67, 64, D, 2, H), 11, batch=5)
+    for T in (8, 38):
+        prompts = np.stack([fhp.TrainingRandom(20 + b).ids(67, T) for b in range(5)])
+        ids, lg = fhp.Sampler.generate(m, prompts, 4, 0.0, 0, None, return_logits=True)
+        for b in (0, 4):
+            rids, rlg = oracle.generate(oc, w, prompts[b], 4, return_logits=True)
+            assert_greedy_parity(ids[b], lg[b], rids, rlg, TOL_F32, f"{T} rows, sequence {b}")
+    m.dispose()
