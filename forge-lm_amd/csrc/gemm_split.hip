@@ -28,8 +28,10 @@
 // results themselves 0.42e-6 and 0.85e-6 (fp32 0.50e-6 and 0.99e-6).  It costs 2-5% of the time.
 //
 // Infinities and NaN: a split of them makes products the fp32 sum would not have (inf *
-// 0), so a block whose sums are not all finite computes its tile again by fp32
-// multiply-adds from memory.  A finite result cannot have met one.
+// 0), so a block whose sums are not all finite computes its tile again on the fp32 matrix
+// cores.  A finite result cannot have met one.  A product of NaN alone takes about twice
+// its time (2048 x 768 x 3072: 69 -> 141 us, with one row of NaN 113; scalar multiply-adds
+// in place of the matrix cores took 5700 in both).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -154,6 +156,16 @@ struct Operand {
 #pragma unroll
         for (int j = 0; j < 8; j++) v[u][j] = 8 * chunk + j < krem ? v[u][j] : 0.f;
     }
+  }
+
+  // the elements as they are, 128 bytes a row: 16-byte chunk c of row r at c ^ (r & 7)
+  __device__ __forceinline__ void store_f32(char* lds, const float (&v)[U][8]) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        *reinterpret_cast<float4*>(lds + (row + 64 * u) * 128 + 16 * ((2 * chunk + q) ^ (row & 7))) =
+            make_float4(v[u][4 * q], v[u][4 * q + 1], v[u][4 * q + 2], v[u][4 * q + 3]);
   }
 
   // `sign`: 0 or the sign bit, flipped into every element
@@ -305,34 +317,63 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   const int rows = min(BM, g.M - m0);
   const bool parts = g.part != nullptr;
   float* const out = parts ? g.part + (size_t)split * g.slots * g.M * g.N : g.y;
-  int bad = 0;
+  // rows and columns past the end may be flagged too: that costs time only
+  bool bad = false;
 #pragma unroll
   for (int i = 0; i < MT; i++)
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
-      const bool in_n = n0 + wn * (BN / 2) + j * 32 + fr < g.N;
+    for (int j = 0; j < NT; j++)
 #pragma unroll
-      for (int r = 0; r < 16; r++)
-        bad |= in_n && wm * (BM / 2) + i * 32 + mfma_acc_row(lane, r) < rows && !(fabsf(acc[0][i][j][r]) < INFINITY);
-    }
+      for (int r = 0; r < 16; r++) bad |= !(fabsf(acc[0][i][j][r]) < INFINITY);
   if (__syncthreads_or(bad)) {
-    // not all finite: the tile by fp32 multiply-adds in k order
-    for (int e = tid; e < BM * BN; e += 256) {
-      const int m = m0 + e / BN, n = n0 + e % BN;
-      if (m >= g.M || n >= g.N) continue;
-      float s = 0.f;
-      for (int k = kb; k < ke; k++)
-        s = fmaf(AKC ? a[(size_t)m * g.K + k] : a[(size_t)k * g.M + m],
-                 BKC ? b[(size_t)n * g.K + k] : b[(size_t)k * g.N + n], s);
-      const size_t at = ((size_t)slot * g.M + m) * g.N + n;
-      if (!parts) {
-        if (g.bias) s += g.bias[n];
-        if (g.gelu) s = gelu_tanh(s);
-        if (g.res) s += g.res[at];
+    // the tile again on the fp32 matrix cores, which give what fp32 arithmetic gives
+    oa.init(a, AKC ? g.K : g.M, g.M, m0, g.K, kb, tid);
+    ob.init(b, BKC ? g.K : g.N, g.N, n0, g.K, kb, tid);
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[0][i][j][r] = 0.f;
+    for (int st = 0; st < nst + (krem != 0); st++) {
+      if (st < nst) {
+        oa.template load<false>(va, true);
+        ob.template load<false>(vb, true);
+      } else {
+        oa.template load<true>(va, true);
+        ob.template load<true>(vb, true);
+        oa.mask(va, krem);
+        ob.mask(vb, krem);
       }
-      out[at] = s;
+      oa.store_f32(As, va);
+      ob.store_f32(As + BM * 128, vb);
+      __syncthreads();
+      // a step's two k are k and k + 16 of the stage: 16 bytes of a row feed four steps
+#pragma unroll
+      for (int kk = 0; kk < SK / 8; kk++) {
+        float4 af[MT], bf[NT];
+        const int at = fr * 128 + 16 * ((4 * fh + kk) ^ (fr & 7));
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          af[i] = *reinterpret_cast<const float4*>(As + (wm * (BM / 2) + i * 32) * 128 + at);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          bf[j] = *reinterpret_cast<const float4*>(As + BM * 128 + (wn * (BN / 2) + j * 32) * 128 + at);
+        auto step = [&](auto pick) {
+#pragma unroll
+          for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+              acc[0][i][j] =
+                  __builtin_amdgcn_mfma_f32_32x32x2f32(pick(af[i]), pick(bf[j]), acc[0][i][j], 0, 0, 0);
+        };
+        step([](const float4& v) { return v.x; });
+        step([](const float4& v) { return v.y; });
+        step([](const float4& v) { return v.z; });
+        step([](const float4& v) { return v.w; });
+      }
+      __syncthreads();
     }
-    return;
   }
   const __amdgpu_buffer_rsrc_t ry = rows_rsrc(out, yrow, rows, g.N, 4);
   const __amdgpu_buffer_rsrc_t rres = !parts && g.res ? rows_rsrc(g.res, yrow, rows, g.N, 4) : ry;

@@ -394,24 +394,34 @@ def test_split_matmul_tiles_and_remainders(fhp, tb, mode, slots, M, K, N):
 
 
 @pytest.mark.gpu
-def test_split_matmul_infinities_and_nan(fhp, tb):
-    """Infinite, NaN and overflowing sums are those of fp32 arithmetic; other outputs stay exact to fp32."""
+@pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("acc", [False, True])
+@pytest.mark.parametrize("M,K,N", [(150, 96, 140), (300, 2049, 130), (1025, 768, 1100), (70, 40, 70)])
+def test_split_matmul_infinities_and_nan(fhp, tb, mode, acc, M, K, N):
+    """Infinite, NaN and overflowing sums are those of fp32 arithmetic; other outputs stay exact to fp32:
+    in one launch, split over K with the odd values in different parts of K, in tiles of 128 rows, and with a
+    K that ends inside a stage."""
     g = np.random.default_rng(5)
-    M, K, N = 150, 96, 140
     a = g.standard_normal((M, K)).astype(np.float32)
     b = g.standard_normal((K, N)).astype(np.float32)
+    prior = g.standard_normal((M, N)).astype(np.float32)
     b[7] = 1.0  # exactly representable in bf16: its lower parts are zero
     a[3, 7] = np.inf
-    a[5, 7], a[5, 8] = np.inf, -np.inf
-    b[8] = 2.0
-    a[9, 2] = np.nan
+    a[5, 7], a[5, K - 1] = np.inf, -np.inf
+    b[K - 1] = 2.0
+    a[9, K - 2] = np.nan
+    b[K // 2, 3] = -np.inf
     a[11, :] = 0.0
     a[11, 20], b[20, 4] = 3.4e38, 3.0  # overflows
     a[12, 21], b[21, :] = 3.4028235e38, 0.5  # rounds to infinity in bf16, is finite in fp32
+    prior[14, 2] = np.inf
     with np.errstate(over="ignore", invalid="ignore"):
-        want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32)
-    y = fhp.Tensor(M, N)
-    tb.MatMulNN(dup(fhp, a, M, K), dup(fhp, b, K, N), y, M, K, N)
+        # 0 * inf where a row of zeros meets b's infinity, as fp32 arithmetic has it
+        want = (a.astype(np.float64) @ b.astype(np.float64) + (prior if acc else 0)).astype(np.float32)
+    ta = dup(fhp, a.T.copy(), K, M) if mode == "tn" else dup(fhp, a, M, K)
+    tn = dup(fhp, b.T.copy(), N, K) if mode == "nt" else dup(fhp, b, K, N)
+    y = dup(fhp, prior, M, N)
+    {"nn": tb.MatMulNN, "nt": tb.MatMulNT, "tn": tb.MatMulTN}[mode](ta, tn, y, M, K, N, accumulate=acc)
     tb.EnsureHostCurrent(y)
     got = y.Data.reshape(M, N)
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
@@ -419,7 +429,38 @@ def test_split_matmul_infinities_and_nan(fhp, tb):
     np.testing.assert_array_equal(got[inf], want[inf])
     ok = np.isfinite(want)
     assert np.all(np.isfinite(got[ok]))
-    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=1e-4)
+    # sums of K standard products: K^0.5 of them in size, K^0.5 roundings of that (row 12's by 2^127)
+    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-5, atol=2.0 ** -24 * 8 * K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
+def test_split_matmul_of_nan_takes_a_few_times_a_finite_product(fhp, tb, mode):
+    """Operands with NaN go through the fp32 matrix cores after the split: twice the time of a finite product.
+    The bound leaves a factor of four for noise (a loop of scalar multiply-adds took 80 times)."""
+    import time
+    M, K, N = 2048, 768, 3072
+    g = np.random.default_rng(6)
+    a, b = g.standard_normal((M, K)).astype(np.float32), g.standard_normal((K, N)).astype(np.float32)
+    fn = {"nn": tb.MatMulNN, "nt": tb.MatMulNT, "tn": tb.MatMulTN}[mode]
+    y = fhp.Tensor(M, N)
+
+    def best(first):
+        a[0, 0] = first
+        a[:, 5] = first
+        ta = dup(fhp, a.T.copy(), K, M) if mode == "tn" else dup(fhp, a, M, K)
+        tn = dup(fhp, b.T.copy(), N, K) if mode == "nt" else dup(fhp, b, K, N)
+        times = []
+        for _ in range(6):
+            t = time.perf_counter()
+            for _ in range(20):
+                fn(ta, tn, y, M, K, N)
+            tb.SumSquares(y)  # waits
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    finite = best(1.0)
+    assert best(np.nan) < 8 * finite
 
 
 @pytest.mark.gpu
