@@ -352,8 +352,8 @@ constexpr int kSplitRows = 32;
 constexpr size_t kPartFloats = (size_t)8 << 20;
 
 template <typename WT>
-bool use_split(int M) {
-  return std::is_same<WT, float>::value && M > kSplitRows;
+bool use_split(int M, int K, int N) {
+  return std::is_same<WT, float>::value && M > kSplitRows && gemm_split_fits(1, M, K, N);
 }
 
 // y = epi(x @ W + b) (+ res) for registry matrix `slot`: the GEMV for up to 4 rows, the MFMA GEMM on the transposed copy above that.
@@ -363,7 +363,7 @@ int linear(fh_session* s, const float* x, int M, int K, size_t slot, int N, cons
   hipStream_t st = s->ctx->stream;
   if (M <= 4) {
     LAUNCH(launch_gemv<WT>(st, x, M, K, s->wt<WT>(slot), N, nullptr, nullptr, 0.f, b, epi, res, y));
-  } else if (use_split<WT>(M)) {
+  } else if (use_split<WT>(M, K, N)) {
     LAUNCH(launch_gemm_split(st, 1, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), 1, M, K, N, b,
                              epi == EPI_GELU, res, y, s->part, s->part_floats, s->ctx->props.multiProcessorCount));
   } else if (K % 32 == 0) {
@@ -389,7 +389,7 @@ int linear_ln(fh_session* s, const float* x, int M, size_t ln, size_t slot, int 
 template <typename WT>
 int linear_parts(fh_session* s, const float* x, int M, int K, size_t slot, int N, int* S) {
   hipStream_t st = s->ctx->stream;
-  if (use_split<WT>(M)) {
+  if (use_split<WT>(M, K, N)) {
     LAUNCH(launch_gemm_split_parts(st, x, reinterpret_cast<const float*>(s->wt<WT>(slot)), M, K, N, s->part,
                                    s->part_floats, s->ctx->props.multiProcessorCount, S));
   } else {

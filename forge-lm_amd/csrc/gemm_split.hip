@@ -416,6 +416,8 @@ struct SplitPlan {
   int bm, bn, splits;
 };
 
+constexpr size_t kMaxBlocks = (size_t)1 << 24;  // of 256 threads
+
 constexpr int kTiles[3][2] = {{128, 128}, {128, 64}, {64, 64}};
 
 size_t split_blocks(int bm, int bn, int slots, int M, int N) {
@@ -440,7 +442,7 @@ SplitPlan split_plan(int slots, int M, int K, int N, size_t part_floats, int cus
   for (int i = 0; i < 3; i++) {
     const double tiles = (double)split_blocks(kTiles[i][0], kTiles[i][1], slots, M, N);
     for (int S : counts) {
-      if (S > 1 && (K < S * 2 * SK || mn * S > (double)part_floats)) break;
+      if (S > 1 && (K < S * 2 * SK || mn * S > (double)part_floats || tiles * S >= (double)kMaxBlocks)) break;
       const double rounds = (double)(((size_t)tiles * S + cus - 1) / cus);
       const int stages = ((K + S - 1) / S + SK - 1) / SK;
       double us = fixed[i] + rounds * round[i] + stages * std::max(alone[i], rounds * unit[i]);
@@ -490,10 +492,10 @@ hipError_t run_split(hipStream_t st, int mode, const float* a, const float* b, i
 }  // namespace
 
 bool gemm_split_fits(int slots, int M, int K, int N) {
-  // 32-bit byte offsets within a tile's rows (KC), a stage's k (RC) and a tile's results,
-  // and at most 2^32 threads in the grid, with room for 32 splits of the smallest tile
-  return slots > 0 && M > 0 && K > 0 && N > 0 && std::max({M, K, N}) < (1 << 21) &&
-         (int64_t)slots * M < (1 << 30) && split_blocks(64, 64, slots, M, N) < (1u << 19);
+  // 32-bit byte offsets: 128 rows of K floats (KC), 32 k of M or N floats (RC) and the 128 rows of N
+  // floats that a tile writes; and a grid below 2^32 threads
+  return slots > 0 && M > 0 && K > 0 && N > 0 && M < (1 << 24) && K < (1 << 22) && N < (1 << 22) &&
+         (int64_t)slots * M < (1 << 30) && split_blocks(64, 64, slots, M, N) < kMaxBlocks;
 }
 
 hipError_t launch_gemm_split(hipStream_t st, int mode, const float* a, const float* b, int slots, int M, int K, int N,

@@ -1245,3 +1245,15 @@ def test_fused_epilogue_split_counts_match_oracle(fhp, oracle, backend, D, H):
             rids, rlg = oracle.generate(oc, w, prompts[b], 4, return_logits=True)
             assert_greedy_parity(ids[b], lg[b], rids, rlg, TOL_F32, f"{T} rows, sequence {b}")
     m.dispose()
+
+
+def test_fp32_windows_of_millions_of_rows(fhp, oracle, backend):
+    """2^21 rows in one window (16384 sequences of 128), past 2^20 and 2^21 tiles and rows of a product."""
+    B, T = 16384, 128
+    m, oc, w = make_model(fhp, oracle, backend, (67, T, 8, 1, 2), 5, batch=B)
+    ids = np.random.default_rng(1).integers(0, 67, (B, T), dtype=np.int32)
+    got = m.forward_last(ids)
+    m.dispose()
+    for b in (0, B // 2 + 1, B - 1):
+        _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
+        assert rel_err(got[b], rlg[0]) <= TOL_F32

@@ -394,6 +394,41 @@ def test_split_matmul_tiles_and_remainders(fhp, tb, mode, slots, M, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode,slots,M,K,N",
+                         [(m, *s) for m in ("nn", "nt", "tn") for s in
+                          [(1, (1 << 21) + 1, 17, 3), (1, 3, (1 << 21) + 7, 5), (1, 2, 18, (1 << 21) + 5),
+                           (1, 2, 1, 1 << 22), (1, 1, 18, 1 << 22)]] + [("nn", 65535, 1, 13, 520)])
+def test_matmul_of_millions(fhp, tb, mode, slots, M, K, N):
+    """Each dimension past 2^21, the scalar kernel past 2^22 columns, and more than 2^19 tiles: against float64
+    at rows, slots and columns of both ends."""
+    g = np.random.default_rng(M % 97 + N % 89)
+
+    def normal(*shape):  # a pattern whose length divides no dimension
+        return np.resize(g.standard_normal(1000003).astype(np.float32), shape)
+
+    a = normal(slots, K, M) if mode == "tn" else normal(slots, M, K)
+    b = normal(slots, N, K) if mode == "nt" else normal(slots, K, N)
+    prior = normal(slots, M, N)
+    fn = {"nn": tb.BatchedMatMulNN, "nt": tb.BatchedMatMulNT, "tn": tb.BatchedMatMulTN}[mode]
+    ta, tn = dup(fhp, a, slots * a.shape[1], a.shape[2]), dup(fhp, b, slots * b.shape[1], b.shape[2])
+    ss = sorted({0, slots // 2, slots - 1})
+    mm = sorted({*range(min(M, 40)), *range(max(0, M - 40), M)})
+    nn = sorted({*range(min(N, 40)), *range(max(0, N - 40), N)})
+    for acc in (False, True):
+        y = dup(fhp, prior, slots * M, N)
+        fn(ta, tn, y, slots, M, K, N, acc)
+        tb.EnsureHostCurrent(y)
+        got = y.Data.reshape(slots, M, N)
+        for s in ss:
+            A = (a[s].T if mode == "tn" else a[s])[mm].astype(np.float64)
+            B = (b[s].T if mode == "nt" else b[s])[:, nn].astype(np.float64)
+            P = prior[s][np.ix_(mm, nn)] if acc else 0
+            err = got[s][np.ix_(mm, nn)] - A @ B - P
+            size = np.linalg.norm(A @ B) + np.linalg.norm(P)
+            assert np.linalg.norm(err) <= 2.0 ** -24 * (2 + np.sqrt(K)) * size
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("acc", [False, True])
 @pytest.mark.parametrize("M,K,N", [(150, 96, 140), (300, 2049, 130), (1025, 768, 1100), (70, 40, 70)])
