@@ -206,11 +206,12 @@ class HipTensorBackend:
     def UnpackQkvHeads(self, q, k, v, dst, batch, T, nHeads, headDim):
         """ITensorBackend.cs:68-76."""
         d = nHeads * headDim
-        if dst.Cols == 3 * d and dst.Length == batch * T * 3 * d:
+        one = min(batch, T, nHeads, headDim) > 0 and 3 * d <= dst.Cols and not any(t is dst for t in (q, k, v))
+        if one and dst.Cols == 3 * d and dst.Length == batch * T * 3 * d:
             self._write(dst)  # the three slices fill it: no zeros to write, no host copy to upload
         else:
             self.Zero(dst)
-        if min(batch, T, nHeads, headDim) > 0 and 3 * d <= dst.Cols and not any(t is dst for t in (q, k, v)):
+        if one:
             pq, pk, pv = self._read(q), self._read(k), self._read(v)
             N.check(N.lib().fh_op_unpack_qkv_heads(self._ctx, pq, pk, pv, self._write(dst, preserve=True), dst.Cols,
                                                    batch, T, nHeads, headDim))

@@ -1031,6 +1031,27 @@ def test_unpack_qkv_zeroes_what_it_does_not_fill(fhp, tb, rows, cols):
 
 
 @pytest.mark.gpu
+def test_unpack_qkv_zeroes_before_calls_out_of_the_ordinary(fhp, tb):
+    """dst zeroed where q is dst itself (its slice is then of zeros), and before sizes that are refused."""
+    g = np.random.default_rng(3)
+    B, T, H, hd = 2, 3, 2, 2
+    k, v = (dup(fhp, g.standard_normal((B * H * T, hd)), B * H * T, hd) for _ in range(2))
+    dst = dup(fhp, np.full((B * T, 12), 5.0), B * T, 12)
+    tb.Scale(dst, 1.0)
+    tb.UnpackQkvHeads(dst, k, v, dst, B, T, H, hd)
+    tb.EnsureHostCurrent(dst)
+    want = np.zeros((B * T, 12), np.float32)
+    for i, t in ((1, k), (2, v)):
+        want[:, 4 * i:4 * i + 4] = t.Data.reshape(B, H, T, hd).transpose(0, 2, 1, 3).reshape(B * T, 4)
+    np.testing.assert_array_equal(dst.Data.reshape(B * T, 12), want)
+    dst = dup(fhp, np.full((B * T, 12), 5.0), B * T, 12)
+    with pytest.raises(Exception, match="head slices"):
+        tb.UnpackQkvHeads(k, k, v, dst, -B, -T, H, hd)
+    tb.EnsureHostCurrent(dst)
+    assert np.all(dst.Data == 0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 100001])
 def test_adamw_lengths(fhp, tb, n):
     """Lengths around the 16-byte groups: every element stepped once, against float64 (a few roundings)."""
