@@ -1129,7 +1129,8 @@ def test_gelu_of_infinities_and_nan(fhp, oracle, tb):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4), (5, 1023), (2, 1028), (9000, 8)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 4), (5, 1023), (2, 1028), (9000, 8), (1100000, 1), (300, 31),
+                                       (70001, 40), (5, 256), (5, 260), (100, 129)])
 def test_add_bias_shapes(fhp, tb, rows, cols):
     """Rows by 16 bytes and by 4, a last strip in part, more rows than block rows: one addition each."""
     g = np.random.default_rng(rows + cols)
@@ -1164,3 +1165,33 @@ def test_pack_qkv_in_one_launch(fhp, tb, hd, extra):
     tb.PackQkvHeads(ts, q, q, v, B, T, H, hd)
     tb.EnsureHostCurrent(q)
     np.testing.assert_array_equal(q.Data.reshape(want[1].shape), want[1])
+
+
+def _pace(tb, f, ref):
+    """Time of f over that of ref, each the best of several runs of 40 calls."""
+    import time
+
+    def best(g):
+        times = []
+        for _ in range(6):
+            t = time.perf_counter()
+            for _ in range(40):
+                g()
+            wait()
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    import forge_hip
+    one = forge_hip.Tensor(1)
+    wait = lambda: tb.SumSquares(one)  # noqa: E731 - the next call that waits for the device
+    best(ref)
+    return best(f) / best(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(1 << 20, 1), (1 << 20, 8), (1 << 18, 31)])
+def test_add_bias_of_narrow_rows_keeps_pace(fhp, tb, rows, cols):
+    """Against AddInPlace of as many elements, which moves half as much again: at most three times its time."""
+    y, src, b = (dup(fhp, np.ones(n), *s) for n, s in ((rows * cols, (rows, cols)), (rows * cols, (rows, cols)),
+                                                      (cols, (cols,))))
+    assert _pace(tb, lambda: tb.AddBias(y, b, rows, cols), lambda: tb.AddInPlace(src, y)) < 3
