@@ -144,26 +144,31 @@ __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, con
 }
 
 // ---- head packing (PackHeads / UnpackHeads, CpuBackend.cs:225-262) ----------------
-// HBM-bound copies.  A block row (blockIdx.y) is one (sequence, head) slot, so a thread
-// divides by the head's width alone, and V (4 where widths, offsets and pointers are
-// multiples of 16 bytes) floats move per load (48 slots of 331 x 64: 5.9 -> 3.4 us; three
-// divisions per float before).  blockIdx.z is one of up to three packed tensors whose columns
-// follow each other (q, k and v in one launch: 4.9 us for three of 4 MB, 3.4 for one).
+// HBM-bound copies.  A thread works within one (sequence, head) slot, so it divides by the head's
+// width alone, and V (4 where widths, offsets and pointers are multiples of 16 bytes) floats move per
+// load (48 slots of 331 x 64: 5.9 -> 3.4 us; three divisions per float before).  `wide` threads of
+// a block share a slot, 256 / wide slots lie side by side: short slots (T of 1) fill a
+// block too (16384 x 4 slots of 1 x 8: 4.4 us, a block to each 30).  blockIdx.z is one of up to three
+// packed tensors whose columns follow each other (q, k and v in one launch: 4.9 us for three of 4 MB,
+// 3.4 for one).  I: 64 bits where a slot or the slots are 2^31 or more.
 struct PackSlices {
   float* packed[3];
 };
-template <int V>
-__global__ __launch_bounds__(256) void k_pack_heads(float* __restrict__ wide, int wide_cols, PackSlices slices,
-                                                    int slots, int T, int H, int hd, int col_base, int unpack) {
-  const unsigned per = hd / V, n = (unsigned)T * per;
+template <int V, typename I>
+__global__ __launch_bounds__(256) void k_pack_heads(float* __restrict__ wide_rows, int wide_cols, PackSlices slices,
+                                                    I slots, int T, int H, int hd, int col_base, unsigned wide,
+                                                    int unpack) {
+  const unsigned per = hd / V, side = 256 / wide, ts = threadIdx.x / wide;
+  if (ts >= side) return;
+  const I n = (I)T * per;
   float* __restrict__ const packed = slices.packed[blockIdx.z];
   const int col = col_base + blockIdx.z * H * hd;
-  for (int s = blockIdx.y; s < slots; s += gridDim.y) {
-    const int q = s / H, h = s % H;
+  for (I s = (I)blockIdx.y * side + ts; s < slots; s += (I)gridDim.y * side) {
+    const I q = s / H, h = s % H;
     const size_t wide0 = (size_t)q * T * wide_cols + col + h * hd, packed0 = (size_t)s * T * hd;
-    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-      const unsigned t = i / per, e = i % per * V;
-      float* const pw = wide + wide0 + (size_t)t * wide_cols + e;
+    for (I i = (I)blockIdx.x * wide + (threadIdx.x - ts * wide); i < n; i += (I)gridDim.x * wide) {
+      const I t = i / per, e = i % per * V;
+      float* const pw = wide_rows + wide0 + (size_t)t * wide_cols + e;
       float* const pp = packed + packed0 + (size_t)i * V;
       if constexpr (V == 4) {
         if (unpack)
@@ -1111,11 +1116,18 @@ int launch_pack(hipStream_t st, float* wide, int wide_cols, const PackSlices& p,
                 int hd, int col_base, int unpack) {
   bool v4 = hd % 4 == 0 && wide_cols % 4 == 0 && col_base % 4 == 0 && aligned16(wide);
   for (int i = 0; i < count; i++) v4 = v4 && aligned16(p.packed[i]);
-  const size_t n = (size_t)T * hd / (v4 ? 4 : 1);
-  const int slots = batch * H;
-  const dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 65535), (unsigned)std::min(slots, 65535), count);
-  hipLaunchKernelGGL(v4 ? k_pack_heads<4> : k_pack_heads<1>, grid, dim3(256), 0, st, wide, wide_cols, p, slots, T, H, hd,
-                     col_base, unpack);
+  const size_t n = (size_t)T * (hd / (v4 ? 4 : 1)), slots = (size_t)batch * H;
+  const unsigned slot_threads = (unsigned)std::min<size_t>(n, 256), side = 256 / slot_threads;
+  const dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 65535),
+                  (unsigned)std::min<size_t>((slots + side - 1) / side, 65535), count);
+  auto launch = [&](auto kernel, auto typed_slots) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, wide, wide_cols, p, typed_slots, T, H, hd, col_base,
+                       slot_threads, unpack);
+  };
+  if (std::max(n, slots) < (size_t)1 << 31)
+    launch(v4 ? k_pack_heads<4, unsigned> : k_pack_heads<1, unsigned>, (unsigned)slots);
+  else
+    launch(v4 ? k_pack_heads<4, size_t> : k_pack_heads<1, size_t>, slots);
   return op_launched(unpack ? "unpack heads" : "pack heads");
 }
 

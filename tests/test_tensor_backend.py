@@ -957,7 +957,8 @@ def test_cross_entropy_vocabulary_widths(fhp, tb, T, V):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,T,H,hd,pad", [(1, 1, 1, 1, 0), (2, 5, 3, 6, 2), (3, 17, 2, 64, 0), (1, 300, 4, 20, 1),
-                                              (2, 9, 5, 8, 4)])
+                                              (2, 9, 5, 8, 4), (701, 1, 3, 8, 0), (40, 1, 5, 7, 3), (30000, 1, 3, 2, 0),
+                                              (5, 4, 3, 256, 4), (3, 129, 3, 4, 0), (2, 256, 2, 1, 0), (2, 257, 2, 1, 0)])
 def test_head_packing_widths(fhp, tb, batch, T, H, hd, pad):
     """Head packing in both directions, by 16-byte and by single loads (odd widths and offsets), exactly."""
     d = H * hd
@@ -1195,3 +1196,13 @@ def test_add_bias_of_narrow_rows_keeps_pace(fhp, tb, rows, cols):
     y, src, b = (dup(fhp, np.ones(n), *s) for n, s in ((rows * cols, (rows, cols)), (rows * cols, (rows, cols)),
                                                       (cols, (cols,))))
     assert _pace(tb, lambda: tb.AddBias(y, b, rows, cols), lambda: tb.AddInPlace(src, y)) < 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,T,H,hd", [(16384, 1, 4, 8), (4096, 1, 12, 64), (2000, 3, 8, 5)])
+def test_head_packing_of_short_slots_keeps_pace(fhp, tb, batch, T, H, hd):
+    """Against Copy of the packed tensor, which moves as much: at most three times its time."""
+    n = batch * T * H * hd
+    src = dup(fhp, np.ones(n), batch * T, H * hd)
+    out, cp = fhp.Tensor(batch * H * T, hd), fhp.Tensor(batch * H * T, hd)
+    assert _pace(tb, lambda: tb.PackHeads(src, out, batch, T, H, hd, 0), lambda: tb.Copy(out, cp)) < 3
