@@ -813,6 +813,37 @@ __global__ __launch_bounds__(1024) void k_ce_forward_row(const float* logits, co
   if (threadIdx.x == 0) nll[t] = ignored ? 0.f : logf(sum) + mx - tl;
 }
 
+// The same for rows of at most 64 VPL columns: a wave to a row, no barrier (with the upload and the
+// loss summed on the device, 65536 x 100: 103 us, 1024 threads to a row 323; 16000 x 300: 46 and 98).
+template <int VPL>
+__global__ __launch_bounds__(256) void k_ce_forward_wave(const float* logits, const int* __restrict__ targets,
+                                                         float* probs, int T, int V, int ignore,
+                                                         float* __restrict__ nll) {
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T) return;
+  const float* lr = logits + (size_t)t * V;
+  float* pr = probs + (size_t)t * V;
+  const int tg = targets[t];
+  const bool ignored = tg == ignore;
+  const float tl = ignored ? 0.f : lr[tg];
+  float v[VPL], mx = -INFINITY, s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPL; i++) v[i] = lane + 64 * i < V ? lr[lane + 64 * i] : -INFINITY;
+#pragma unroll
+  for (int i = 0; i < VPL; i++) mx = fmaxf(mx, v[i]);
+  mx = wave_max_dpp(mx);
+#pragma unroll
+  for (int i = 0; i < VPL; i++) {
+    v[i] = lane + 64 * i < V ? expf(v[i] - mx) : 0.f;
+    s += v[i];
+  }
+  const float sum = wave_sum_dpp(s), inv = 1.f / sum;
+#pragma unroll
+  for (int i = 0; i < VPL; i++)
+    if (lane + 64 * i < V) pr[lane + 64 * i] = v[i] * inv;
+  if (lane == 0) nll[t] = ignored ? 0.f : logf(sum) + mx - tl;
+}
+
 // acc (double, device) += sum of the T per-position terms, by one block in double (fixed order)
 __global__ __launch_bounds__(256) void k_ce_accumulate(const float* __restrict__ nll, int T, double* __restrict__ acc) {
   __shared__ double red[256];
@@ -825,28 +856,59 @@ __global__ __launch_bounds__(256) void k_ce_accumulate(const float* __restrict__
 // HBM-bound: a block takes kCeCols columns of a position (blockIdx.x; blockIdx.y its part of
 // the vocabulary), so no element divides by V and 8 loads per thread are in flight (500 x
 // 16257: 21 -> 13 us).
-constexpr int kCeCols = 2048;
+constexpr unsigned kCeCols = 2048;
 __global__ __launch_bounds__(256) void k_ce_backward(const float* probs, const int* __restrict__ targets, float* dl,
-                                                     int V, int ignore, float scale) {
-  const int t = blockIdx.x, tg = targets[t];
-  const size_t at = (size_t)t * V;
-  for (int c0 = blockIdx.y * kCeCols; c0 < V; c0 += gridDim.y * kCeCols) {
-    float p[8];
+                                                     unsigned T, unsigned V, int ignore, float scale) {
+  for (unsigned t = blockIdx.x; t < T; t += gridDim.x) {
+    const int tg = targets[t];
+    const size_t at = (size_t)t * V;
+    for (unsigned c0 = blockIdx.y * kCeCols; c0 < V; c0 += gridDim.y * kCeCols) {
+      float p[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int c = c0 + threadIdx.x + 256 * i;
-      p[i] = tg != ignore && c < V ? probs[at + c] : 0.f;
-    }
+      for (int i = 0; i < 8; i++) {
+        const unsigned c = c0 + threadIdx.x + 256 * i;
+        p[i] = tg != ignore && c < V ? probs[at + c] : 0.f;
+      }
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int c = c0 + threadIdx.x + 256 * i;
-      float g = p[i] * scale;
-      if (tg == ignore)
-        g = 0.f;
-      else if (c == tg)
-        g = g - scale;
-      if (c < V) dl[at + c] = g;
+      for (int i = 0; i < 8; i++) {
+        const unsigned c = c0 + threadIdx.x + 256 * i;
+        float g = p[i] * scale;
+        if (tg == ignore)
+          g = 0.f;
+        else if ((int)c == tg)
+          g = g - scale;
+        if (c < V) dl[at + c] = g;
+      }
     }
+  }
+}
+
+// The same for V <= kCeFlat: a block takes kCeFlatPer elements of the positions one after the other,
+// with a 32-bit division per element (with the targets' upload, 262144 x 10: 117 us, a block to each
+// position 165; 65536 x 100: 40 and 59; 8000 x 600: 26.7 and 28.1; 4096 x 1024: 11.9 and 11.3).
+constexpr int kCeFlat = 768, kCeFlatPer = 2048;
+__global__ __launch_bounds__(256) void k_ce_backward_flat(const float* probs, const int* __restrict__ targets, float* dl,
+                                                          size_t n, int V, int ignore, float scale) {
+  const size_t base = (size_t)blockIdx.x * kCeFlatPer, t0 = base / V;
+  const unsigned c0 = (unsigned)(base - t0 * V), left = (unsigned)min((size_t)kCeFlatPer, n - base);
+  float p[8];
+  int tg[8];
+  unsigned c[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const unsigned j = min(threadIdx.x + 256u * i, left - 1), t = (c0 + j) / V;
+    c[i] = c0 + j - t * V;
+    tg[i] = targets[t0 + t];
+    p[i] = probs[base + j];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    float g = p[i] * scale;
+    if (tg[i] == ignore)
+      g = 0.f;
+    else if ((int)c[i] == tg[i])
+      g = g - scale;
+    if (threadIdx.x + 256u * i < left) dl[base + threadIdx.x + 256u * i] = g;
   }
 }
 
@@ -1442,14 +1504,17 @@ int fh_op_cross_entropy_forward(fh_context* c, const void* logits, const int32_t
   FH_TRY(copy_ints(c, ops_, targets, (size_t)T, dt));
   const float* lg = static_cast<const float*>(logits);
   float* pr = static_cast<float*>(probs);
-  if (V <= 1024 * 4)
+  if (V <= kRowWaveCols)
+    ROW_WAVES(k_ce_forward_wave, V,
+              <<<dim3((unsigned)(((size_t)T + 3) / 4)), dim3(256), 0, st_>>>(lg, dt, pr, T, V, ignore_index, nll));
+  else if (V > 1024 * 32 || T >= 1 << 22)  // (a grid of 1024-thread blocks ends at 2^32 threads)
+    hipLaunchKernelGGL(k_ce_forward, dim3(T), dim3(256), 0, st_, lg, dt, pr, V, ignore_index, nll);
+  else if (V <= 1024 * 4)
     hipLaunchKernelGGL(k_ce_forward_row<4>, dim3(T), dim3(1024), 0, st_, lg, dt, pr, V, ignore_index, nll);
   else if (V <= 1024 * 16)
     hipLaunchKernelGGL(k_ce_forward_row<16>, dim3(T), dim3(1024), 0, st_, lg, dt, pr, V, ignore_index, nll);
-  else if (V <= 1024 * 32)
-    hipLaunchKernelGGL(k_ce_forward_row<32>, dim3(T), dim3(1024), 0, st_, lg, dt, pr, V, ignore_index, nll);
   else
-    hipLaunchKernelGGL(k_ce_forward, dim3(T), dim3(256), 0, st_, lg, dt, pr, V, ignore_index, nll);
+    hipLaunchKernelGGL(k_ce_forward_row<32>, dim3(T), dim3(1024), 0, st_, lg, dt, pr, V, ignore_index, nll);
   FH_TRY(op_launched("cross-entropy forward"));
   if (ops_->accumulating) {
     // the loss stays on the device until the accumulation ends (ITensorBackend.cs:154-161)
@@ -1507,9 +1572,15 @@ int fh_op_cross_entropy_backward(fh_context* c, const void* probs, const int32_t
   }
   int* dt = nullptr;
   FH_TRY(upload_ints(c, ops_, targets, (size_t)T, &dt));
-  hipLaunchKernelGGL(k_ce_backward, dim3(T, std::min((V + kCeCols - 1) / kCeCols, 65535)), dim3(256), 0, st_,
-                     static_cast<const float*>(probs), dt, static_cast<float*>(dlogits), V, ignore_index,
-                     1.f / (float)count);
+  const float* pr = static_cast<const float*>(probs);
+  float* dl = static_cast<float*>(dlogits);
+  const size_t blocks = (n + kCeFlatPer - 1) / kCeFlatPer;
+  if (V <= kCeFlat && blocks < (1u << 24))
+    hipLaunchKernelGGL(k_ce_backward_flat, dim3((unsigned)blocks), dim3(256), 0, st_, pr, dt, dl, n, V, ignore_index,
+                       1.f / (float)count);
+  else
+    hipLaunchKernelGGL(k_ce_backward, dim3(std::min(T, 1 << 23), std::min(((unsigned)V + kCeCols - 1) / kCeCols, 65535u)),
+                       dim3(256), 0, st_, pr, dt, dl, (unsigned)T, (unsigned)V, ignore_index, 1.f / (float)count);
   return op_launched("cross-entropy backward");
 }
 

@@ -925,7 +925,8 @@ def test_row_kernels_widths(fhp, tb, rows, cols):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,V", [(3, 1), (2, 1023), (5, 4096), (3, 4097), (4, 16385), (2, 32768), (2, 32769)])
+@pytest.mark.parametrize("T,V", [(3, 1), (2100, 2), (700, 65), (9, 128), (4099, 10), (5, 769), (3, 1024), (3, 1025),
+                                 (2, 1023), (5, 4096), (3, 4097), (4, 16385), (2, 32768), (2, 32769)])
 def test_cross_entropy_vocabulary_widths(fhp, tb, T, V):
     """CrossEntropy forward (in place) and backward at the edges of the vocabularies that pick a kernel."""
     g = np.random.default_rng(T + V)
@@ -1206,3 +1207,46 @@ def test_head_packing_of_short_slots_keeps_pace(fhp, tb, batch, T, H, hd):
     src = dup(fhp, np.ones(n), batch * T, H * hd)
     out, cp = fhp.Tensor(batch * H * T, hd), fhp.Tensor(batch * H * T, hd)
     assert _pace(tb, lambda: tb.PackHeads(src, out, batch, T, H, hd, 0), lambda: tb.Copy(out, cp)) < 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,V", [(1 << 18, 10), (65536, 100)])
+def test_cross_entropy_of_narrow_vocabularies_keeps_pace(fhp, tb, T, V):
+    """Forward (the loss accumulated on the device) and backward against Copy of the logits, with the targets'
+    upload in both: at most three times its time."""
+    lg, pr = dup(fhp, np.zeros(T * V), T, V), fhp.Tensor(T, V)
+    tg = np.zeros(T, np.int32)
+    tab, up = dup(fhp, np.zeros(4), 4, 1), fhp.Tensor(T, 1)
+
+    def ref():
+        tb.EmbeddingForward(tab, tg, up, 1)  # the same upload
+        tb.Copy(lg, pr)
+
+    tb.BeginLossAccumulation()
+    assert _pace(tb, lambda: tb.CrossEntropyForward(lg, tg, pr, T, V, -1), ref) < 3
+    tb.EndLossAccumulation()
+    assert _pace(tb, lambda: tb.CrossEntropyBackward(pr, tg, lg, T, V, -1), ref) < 3
+
+
+@pytest.mark.gpu
+def test_cross_entropy_of_millions_of_positions(fhp, tb):
+    """2^22 positions and more, narrow and (in place on 17 GB) wider than a wave's registers: uniform rows."""
+    from forge_hip import _native as N
+    import ctypes
+    for T, V in ((5000001, 3), ((1 << 22) + 1, 1025)):
+        buf = fhp.DeviceBuffer(tb.backend, 4 * T * V)
+        N.check(N.lib().fh_op_zero(tb._ctx, buf.ptr, T * V))
+        tg = np.zeros(T, np.int32)
+        loss = ctypes.c_float()
+        N.check(N.lib().fh_op_cross_entropy_forward(tb._ctx, buf.ptr, tg.ctypes.data, buf.ptr, T, V, -1,
+                                                    ctypes.byref(loss)))
+        assert abs(loss.value - np.log(V)) < 1e-5
+        N.check(N.lib().fh_op_cross_entropy_backward(tb._ctx, buf.ptr, tg.ctypes.data, buf.ptr, T, V, -1))
+        for row in (0, T // 2, T - 1):
+            got = np.empty(V, np.float32)
+            N.check(N.lib().fh_buffer_read(tb._ctx, got.ctypes.data, ctypes.c_void_p(buf.ptr.value + 4 * row * V),
+                                           4 * V))
+            want = np.full(V, 1 / V / T)
+            want[0] -= 1 / T
+            np.testing.assert_allclose(got, want, rtol=1e-5, atol=0)
+        buf.free()
