@@ -80,9 +80,10 @@ unsigned grid_for(size_t n) { return (unsigned)std::min<size_t>((n + kT - 1) / k
 unsigned grid_vec(size_t n, bool v4) { return grid_for(v4 ? (n + 3) / 4 : n); }
 
 // ---- matmuls: y[s] (+)= op(a[s]) @ op(b[s]), 64x64 tiles, k steps of 16 ------------
-// for sizes that the split GEMM does not take (gemm_split_fits), with 64-bit offsets
-// MODE 0 NN (a [M,K], b [K,N]), 1 NT (b [N,K]), 2 TN (a [K,M]).
-template <int MODE>
+// for few k, and for sizes that the split GEMM does not take (gemm_split_fits), with 64-bit offsets
+// MODE 0 NN (a [M,K], b [K,N]), 1 NT (b [N,K]), 2 TN (a [K,M]).  Sums in S: the few products of
+// fp32 elements are exact in double and hide behind the stores, so such a result is rounded once.
+template <int MODE, typename S>
 __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, const float* __restrict__ b,
                                                 float* __restrict__ y, int M, int K, int N, int acc) {
   __shared__ float As[16][65];
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, con
   y += (size_t)s * M * N;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float c[4][4] = {};
+  S c[4][4] = {};
   for (int k0 = 0; k0 < K; k0 += 16) {
     for (int i = threadIdx.x; i < 1024; i += 256) {
       // A tile [16 k][64 m], B tile [16 k][64 n]
@@ -115,17 +116,25 @@ __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, con
       Bs[kb][nn] = (gn < N && gk2 < K) ? (MODE == 1 ? b[(size_t)gn * K + gk2] : b[(size_t)gk2 * N + gn]) : 0.f;
     }
     __syncthreads();
+    auto steps = [&](int from) {
 #pragma unroll
-    for (int kk = 0; kk < 16; kk++) {
-      float av[4], bv[4];
+      for (int kk = 0; kk < 4; kk++) {
+        S av[4], bv[4];
 #pragma unroll
-      for (int i = 0; i < 4; i++) av[i] = As[kk][ty + 16 * i];
+        for (int i = 0; i < 4; i++) av[i] = As[from + kk][ty + 16 * i];
 #pragma unroll
-      for (int j = 0; j < 4; j++) bv[j] = Bs[kk][tx + 16 * j];
+        for (int j = 0; j < 4; j++) bv[j] = Bs[from + kk][tx + 16 * j];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) c[i][j] = fmaf(av[i], bv[j], c[i][j]);
+          for (int j = 0; j < 4; j++) c[i][j] = fma(av[i], bv[j], c[i][j]);
+      }
+    };
+    steps(0);
+    if (sizeof(S) == 4 || k0 + 4 < K) steps(4);
+    if (sizeof(S) == 4 || k0 + 8 < K) {
+      steps(8);
+      steps(12);
     }
     __syncthreads();
   }
@@ -138,7 +147,7 @@ __global__ __launch_bounds__(256) void k_matmul(const float* __restrict__ a, con
       const int n = n0 + tx + 16 * j;
       if (n >= N) continue;
       float& o = y[(size_t)m * N + n];
-      o = acc ? o + c[i][j] : c[i][j];
+      o = acc ? o + (float)c[i][j] : (float)c[i][j];
     }
   }
 }
@@ -1148,7 +1157,12 @@ int matmul_common(fh_context* c, int mode, const void* a, const void* b, void* y
   OPS_PROLOGUE(c);
   OPS_ARG(a && b && y, "null buffer");
   OPS_ARG(slots > 0 && slots <= 65535 && M > 0 && K > 0 && N > 0, "slots (at most 65535), M, K and N must be positive");
-  if (gemm_split_fits(slots, M, K, N)) {
+  // Few k: the split GEMM's stage of 32 is mostly padding, and its results at K 1 are not all rounded
+  // right.  Where y is added to, its wider tiles make up for that unless y is small (us, this kernel and
+  // the split GEMM: 4096 x 1 x 4096 15.1 and 19.4, K 8 18.6 and 19.3, K 12 24 and 19.5; 65535 slots of
+  // 8 x 8 x 8 134 and 200; adding to 48 slots of 331 x 8 x 331 17 and 11).
+  const bool few = M < 1 << 22 && (K == 1 || (K <= 8 && (!acc || (size_t)M * N <= 1024)));
+  if (!few && gemm_split_fits(slots, M, K, N)) {
     const int cus = context_cus(c);
     const size_t pf = gemm_split_part_floats(slots, M, K, N, kSplitPartFloats, cus);
     void* part = nullptr;
@@ -1158,17 +1172,19 @@ int matmul_common(fh_context* c, int mode, const void* a, const void* b, void* y
                               static_cast<float*>(part), pf, cus));
     return FH_OK;
   }
-  // sizes past the split GEMM's 32-bit offsets
   dim3 grid((N + 63) / 64, (M + 63) / 64, slots);
   const float* fa = static_cast<const float*>(a);
   const float* fb = static_cast<const float*>(b);
   float* fy = static_cast<float*>(y);
   if (mode == 0)
-    hipLaunchKernelGGL(k_matmul<0>, grid, dim3(256), 0, st_, fa, fb, fy, M, K, N, acc);
+    hipLaunchKernelGGL((few ? k_matmul<0, double> : k_matmul<0, float>), grid, dim3(256), 0, st_, fa, fb, fy, M, K, N,
+                       acc);
   else if (mode == 1)
-    hipLaunchKernelGGL(k_matmul<1>, grid, dim3(256), 0, st_, fa, fb, fy, M, K, N, acc);
+    hipLaunchKernelGGL((few ? k_matmul<1, double> : k_matmul<1, float>), grid, dim3(256), 0, st_, fa, fb, fy, M, K, N,
+                       acc);
   else
-    hipLaunchKernelGGL(k_matmul<2>, grid, dim3(256), 0, st_, fa, fb, fy, M, K, N, acc);
+    hipLaunchKernelGGL((few ? k_matmul<2, double> : k_matmul<2, float>), grid, dim3(256), 0, st_, fa, fb, fy, M, K, N,
+                       acc);
   return op_launched("matmul");
 }
 

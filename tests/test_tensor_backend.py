@@ -394,6 +394,34 @@ def test_split_matmul_tiles_and_remainders(fhp, tb, mode, slots, M, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("slots,M,K,N", [(1, 300, 1, 517), (3, 65, 2, 64), (1, 63, 7, 130), (700, 8, 8, 8),
+                                         (2, 200, 8, 90), (1, 70, 4, 70), (1, 70, 5, 70)])
+def test_matmul_of_few_k_rounds_once(fhp, tb, mode, slots, M, K, N):
+    """Up to 8 products to a sum: within half an ulp of float64; accumulated, within one of both terms."""
+    g = np.random.default_rng(M + K)
+    a = g.standard_normal((slots, K, M) if mode == "tn" else (slots, M, K)).astype(np.float32)
+    b = g.standard_normal((slots, N, K) if mode == "nt" else (slots, K, N)).astype(np.float32)
+    prior = g.standard_normal((slots, M, N)).astype(np.float32)
+    want = (a.transpose(0, 2, 1) if mode == "tn" else a).astype(np.float64) @ \
+        (b.transpose(0, 2, 1) if mode == "nt" else b).astype(np.float64)
+    fn = {"nn": tb.BatchedMatMulNN, "nt": tb.BatchedMatMulNT, "tn": tb.BatchedMatMulTN}[mode]
+    for acc in (False, True):
+        y = dup(fhp, prior, slots * M, N)
+        fn(dup(fhp, a, slots * a.shape[1], a.shape[2]), dup(fhp, b, slots * b.shape[1], b.shape[2]), y, slots, M, K, N,
+           acc)
+        tb.EnsureHostCurrent(y)
+        err = np.abs(y.Data.reshape(want.shape) - want - (prior if acc else 0))
+        if not acc:
+            assert np.all(err <= 2.0 ** -24 * (1 + 1e-6) * np.abs(want))
+        elif K == 1:
+            assert np.all(err <= 2.0 ** -24 * (1 + 1e-6) * (2 * np.abs(want) + np.abs(prior)))
+        else:  # the split GEMM where the result is wide: K roundings
+            size = np.abs(a).max() * np.abs(b).max() * K + np.abs(prior)
+            assert np.all(err <= 2.0 ** -24 * (K + 2) * size)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode,slots,M,K,N",
                          [(m, *s) for m in ("nn", "nt", "tn") for s in
                           [(1, (1 << 21) + 1, 17, 3), (1, 3, (1 << 21) + 7, 5), (1, 2, 18, (1 << 21) + 5),
