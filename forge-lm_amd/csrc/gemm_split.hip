@@ -32,6 +32,14 @@
 // cores.  A finite result cannot have met one.  A product of NaN alone takes about twice
 // its time (2048 x 768 x 3072: 69 -> 141 us, with one row of NaN 113; scalar multiply-adds
 // in place of the matrix cores took 5700 in both).
+//
+// Small elements: bf16 ends at 2^-133 as fp32 does at 2^-149, so the three parts hold less than
+// 24 bits of an element below 2^-111 (sums of elements near 2^-118 came out 9e-6 off, near 2^-126
+// 2e-3).  What is lost is at most 2^-134 of the other
+// element, so it shows where the sum itself is tiny: a block with a sum below 2^-80 that is not
+// zero computes its tile again as well, which keeps fp32's precision for other elements up to
+// 2^29 / K^0.5.  The test costs 0.5-2% of a product of few stages (48 x 331 x 64 x 331: 16.3 ->
+// 16.6 us).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -324,7 +332,10 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) bad |= !(fabsf(acc[0][i][j][r]) < INFINITY);
+      for (int r = 0; r < 16; r++) {
+        const float x = fabsf(acc[0][i][j][r]);
+        bad |= !(x < INFINITY) || (x < 0x1p-80f && x != 0.f);
+      }
   if (__syncthreads_or(bad)) {
     // the tile again on the fp32 matrix cores, which give what fp32 arithmetic gives
     oa.init(a, AKC ? g.K : g.M, g.M, m0, g.K, kb, tid);

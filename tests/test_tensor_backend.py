@@ -497,6 +497,27 @@ def test_split_matmul_infinities_and_nan(fhp, tb, mode, acc, M, K, N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (300, 2049, 130), (1025, 768, 1100)])
+@pytest.mark.parametrize("exponent", [-60, -85, -108, -112, -118, -126])
+def test_split_matmul_of_tiny_elements(fhp, tb, M, K, N, exponent):
+    """Elements near the bottom of the normal range, on the left or the right, beside ordinary ones: the bound of
+    ordinary elements, and a zero row stays zero.  (Products below 2^-126 are subnormal: multiples of 2^-149.)"""
+    g = np.random.default_rng(K - exponent)
+    a, b = g.standard_normal((M, K)).astype(np.float32), g.standard_normal((K, N)).astype(np.float32)
+    tiny = np.float32(2.0) ** exponent
+    for ta, tn in ((a * tiny, b), (a, b * tiny)):
+        ta[5] = 0
+        want = ta.astype(np.float64) @ tn.astype(np.float64)
+        y = fhp.Tensor(M, N)
+        tb.MatMulNN(dup(fhp, ta, M, K), dup(fhp, tn, K, N), y, M, K, N)
+        tb.EnsureHostCurrent(y)
+        got = y.Data.reshape(M, N)
+        assert np.all(got[5] == 0)
+        err = np.linalg.norm(got - want)
+        assert err <= 2.0 ** -24 * (2 + np.sqrt(K)) * np.linalg.norm(want) + np.sqrt(M * N * K) * 2.0 ** -149, err
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["nn", "nt", "tn"])
 def test_split_matmul_of_nan_takes_a_few_times_a_finite_product(fhp, tb, mode):
     """Operands with NaN go through the fp32 matrix cores after the split: twice the time of a finite product.
