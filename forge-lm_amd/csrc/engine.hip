@@ -347,7 +347,7 @@ int check_launch(hipError_t e, const char* what) {
 // GEMM, whose 32-row tile pads less (a 98M window of 20 rows 0.69 against 0.77 ms; of 66
 // rows 0.93 against 1.05, of 333 1.69 against 1.89, of 1024 3.04 against 3.91)
 constexpr int kSplitRows = 32;
-// room for the partial sums of a split K in fp32 sessions, 32 MB (8 MB: 1024 rows 3.19 ms,
+// room for the partial sums of a split K in fp32 sessions, at most 32 MB (8 MB: 1024 rows 3.19 ms,
 // 3 x 700 rows 4.10 against 3.84; 64 MB no faster)
 constexpr size_t kPartFloats = (size_t)8 << 20;
 
@@ -1237,13 +1237,14 @@ int fh_session_create(fh_context* c, const fh_model_desc* desc, fh_session** out
   sp->vc = vc;
   const size_t rows = (size_t)B * C;
   const int maxc = (C + 63) / 64;
-  // split-K partials: the GEMV path (up to 64 splits of 4 rows), the MFMA GEMM's
-  // small-M split (up to 8 splits of 64 rows of the widest layer), and at least
-  // one unsplit product of every decode row (the batched decode's split GEMMs need
+  // split-K partials: the MFMA GEMM's small-M split (up to 8 splits of 64 rows of the widest layer),
+  // and at least one unsplit product of every decode row (the batched decode's split GEMMs need
   // B x 3D; the split count shrinks to what fits).  short_floats also bounds the windows
-  // whose reductions carry the kernels after them; fp32 sessions have more room for splits
-  sp->short_floats = std::max({(size_t)64 * 4 * 4 * D, (size_t)8 * 64 * 4 * D, (size_t)B * 4 * D});
-  sp->part_floats = std::max(sp->short_floats, desc->dtype == FH_DTYPE_F32 ? kPartFloats : 0);
+  // whose reductions carry the kernels after them; fp32 sessions have more room for the split
+  // GEMM's, as far as their windows can use it (K / 64 splits of M N floats, K N at most 4 D^2)
+  sp->short_floats = std::max((size_t)8 * 64 * 4 * D, (size_t)B * 4 * D);
+  sp->part_floats = std::max(sp->short_floats,
+                             desc->dtype == FH_DTYPE_F32 ? std::min(kPartFloats, rows * D * D / 16) : 0);
   if ((rc = dev_alloc(&sp->x, rows * D)) || (rc = dev_alloc(&sp->x2, rows * D)) || (rc = dev_alloc(&sp->xn, rows * D)) ||
       (rc = dev_alloc(&sp->qkv, rows * 3 * D)) || (rc = dev_alloc(&sp->o, rows * D)) ||
       (rc = dev_alloc(&sp->h, rows * 4 * D)) || (rc = dev_alloc(&sp->part, sp->part_floats)) ||

@@ -1257,3 +1257,18 @@ def test_fp32_windows_of_millions_of_rows(fhp, oracle, backend):
     for b in (0, B // 2 + 1, B - 1):
         _, rlg = oracle.generate(oc, w, ids[b], 1, return_logits=True)
         assert rel_err(got[b], rlg[0]) <= TOL_F32
+
+
+def test_session_of_a_small_model_takes_little_memory(fhp, oracle):
+    """4 layers of d 128 with 128 positions: weights of 5 MB twice over, caches and activations of 2 MB, a few
+    allocations of a page each; no room for partial sums that its windows cannot use."""
+    be = fhp.HipBackend(0)
+    warm = fhp.GptModel(fhp.ModelConfig(67, 16, 8, 1, 2), be)
+    free = be.memory()[0]
+    m = fhp.GptModel(fhp.ModelConfig(2256, 128, 128, 4, 4), be)
+    used = free - be.memory()[0]
+    print(used)
+    m.dispose()
+    warm.dispose()
+    be.dispose()
+    assert used < 24 << 20
