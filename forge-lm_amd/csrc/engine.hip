@@ -643,6 +643,10 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
       // operand load was measured slower (each mlp.proj block re-reads 8 partials
       // of its A chunk: 19 MB per layer)
       const int cus = s->ctx->props.multiProcessorCount;
+      // up to 64 rows in one row of tiles: more splits than short_floats holds cost the kernels that sum
+      // them more than the GEMMs gain (d 1024, 2 layers, 64 rows: 220 us a step, with all of part 245);
+      // of more rows they are too few without (128 rows: 355 against 371, d 768 266 against 307)
+      const size_t parts = B <= 64 ? s->short_floats : s->part_floats;
       // fp32 batches of up to 32 rows: mlp.fc on the skinny GEMM, its bias and GELU
       // in the same launch (8.2 us against 6.1 + 4.4 for the split-K GEMM and its
       // reduction at C4).  qkv and mlp.proj stay split-K: their partials are summed by
@@ -655,7 +659,7 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
         WT* vc = reinterpret_cast<WT*>(s->vc) + (size_t)l * s->kv_layer;
         int S = 0;
         LAUNCH(launch_gemm_mfma_split<WT>(st, s->xn, B, D, s->wt<WT>(s->idx_blk(l, 2)), 3 * D, s->part,
-                                          s->part_floats, cus, &S));
+                                          parts, cus, &S));
         // the attention sums the qkv partials itself and stores the new K/V rows
         const QkvParts qp{s->part, S, B, s->v(s->idx_blk(l, 3))};
         LAUNCH(launch_attn_decode_wide<WT>(st, src, nullptr, B, D, H, C, kc, vc, s->apart, s->o, false, &qp));
@@ -668,7 +672,7 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
         ao.chunk = kAttnDecodeChunk;
         ao.maxc = (C + kAttnDecodeChunk - 1) / kAttnDecodeChunk;
         LAUNCH(launch_gemm_mfma_split<WT>(st, s->apart, B, D, s->wt<WT>(s->idx_blk(l, 4)), D, s->part,
-                                          s->part_floats, cus, &S, &ao));
+                                          parts, cus, &S, &ao));
         LAUNCH(launch_epilogue_ln(st, s->part, S, B, D, s->v(s->idx_blk(l, 5)), s->x, s->x2, s->v(s->idx_blk(l, 6)),
                                   s->v(s->idx_blk(l, 7)), s->xn, 1e-5f));
         if (skinny)
@@ -678,7 +682,7 @@ int enqueue_layers_decode(fh_session* s, RowSrc src) {
           FH_TRY(linear<WT>(s, s->xn, B, D, s->idx_blk(l, 8), 4 * D, s->v(s->idx_blk(l, 9)), EPI_GELU, nullptr,
                             s->h));
         LAUNCH(launch_gemm_mfma_split<WT>(st, s->h, B, 4 * D, s->wt<WT>(s->idx_blk(l, 10)), D, s->part,
-                                          s->part_floats, cus, &S));
+                                          parts, cus, &S));
         const size_t ln = l + 1 < L ? s->idx_blk(l + 1, 0) : s->idx_lnf();
         LAUNCH(launch_epilogue_ln(st, s->part, S, B, D, s->v(s->idx_blk(l, 11)), s->x2, s->x, s->v(ln),
                                   s->v(ln + 1), s->xn, 1e-5f));

@@ -1272,3 +1272,15 @@ def test_session_of_a_small_model_takes_little_memory(fhp, oracle):
     warm.dispose()
     be.dispose()
     assert used < 24 << 20
+
+
+@pytest.mark.parametrize("B", [33, 64, 65])
+def test_batched_decode_splits_match_oracle(fhp, oracle, backend, B):
+    """Decode of a d-1024 batch on both sides of the 64 rows that bound its K splits."""
+    m, oc, w = make_model(fhp, oracle, backend, (67, 32, 1024, 1, 16), 11, batch=B)
+    prompts = np.stack([fhp.TrainingRandom(20 + b).ids(67, 7) for b in range(B)])
+    ids, lg = fhp.Sampler.generate(m, prompts, 4, 0.0, 0, None, return_logits=True)
+    m.dispose()
+    for b in (0, B - 1):
+        rids, rlg = oracle.generate(oc, w, prompts[b], 4, return_logits=True)
+        assert_greedy_parity(ids[b], lg[b], rids, rlg, TOL_F32, f"sequence {b}")
