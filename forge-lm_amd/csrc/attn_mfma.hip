@@ -562,17 +562,17 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill_bf16(const bf16_t* __re
 
 template <typename KT, typename OT>
 hipError_t launch_attn_prefill_mfma(hipStream_t st, const float* qkv, int B, int T, int d, int H, int ctx,
-                                    const KT* kcache, const KT* vcache, OT* o) {
+                                    const KT* kcache, const KT* vcache, OT* o, int cus) {
   if (B <= 0 || T <= 0 || T > ctx || H <= 0 || d != H * HD || !qkv || !kcache || !vcache || !o ||
       (size_t)T * HD * sizeof(KT) > 0x7fffffffu)
     return hipErrorInvalidValue;
   const int blocks = (T + BQ - 1) / BQ * H * B;
   if constexpr (sizeof(KT) == 4) {
-    // below two 128-query blocks per CU the waves are too few (ms per forward of the 98M shape,
+    // up to two 128-query blocks per CU the waves are too few (ms per forward of the 98M shape,
     // 128-query blocks against 32-query ones: 333 rows 1.68 / 1.42, 1024 rows 2.92 / 2.34, 3 x 700
     // 3.75 / 3.54, 16 x 200 4.33 / 4.31); above, sharing a K/V tile in LDS wins (8 x 1024 10.4 /
     // 10.6, 32 x 512 17.2 / 17.6)
-    if (blocks <= 512) {
+    if (blocks <= 2 * (cus > 0 ? cus : 256)) {
       hipLaunchKernelGGL(k_attn_prefill_keys, dim3((T + KQ - 1) / KQ * H * B), dim3(256), 0, st, qkv, 3 * d, T, d, H,
                          ctx, kcache, vcache, o);
       return hipGetLastError();
@@ -594,10 +594,10 @@ hipError_t launch_attn_prefill_mfma_q16(hipStream_t st, const bf16_t* q, int B, 
 }
 
 template hipError_t launch_attn_prefill_mfma<float, float>(hipStream_t, const float*, int, int, int, int, int,
-                                                           const float*, const float*, float*);
+                                                           const float*, const float*, float*, int);
 template hipError_t launch_attn_prefill_mfma<bf16_t, float>(hipStream_t, const float*, int, int, int, int, int,
-                                                            const bf16_t*, const bf16_t*, float*);
+                                                            const bf16_t*, const bf16_t*, float*, int);
 template hipError_t launch_attn_prefill_mfma<bf16_t, bf16_t>(hipStream_t, const float*, int, int, int, int, int,
-                                                             const bf16_t*, const bf16_t*, bf16_t*);
+                                                             const bf16_t*, const bf16_t*, bf16_t*, int);
 
 }  // namespace fh

@@ -566,7 +566,8 @@ int enqueue_layers_window(fh_session* s, int T, RowSrc src, LastRows* last) {
       LAUNCH(launch_epilogue_qkv<WT>(st, s->part, S, M, D, s->v(s->idx_blk(l, 3)), s->qkv, src, T, H, C, kc, vc));
       if (tail && l + 1 == L) return enqueue_last_rows<WT, float>(s, T, src, l, s->qkv, 3 * D, last);
       if (D == 64 * H)
-        LAUNCH((launch_attn_prefill_mfma<WT, float>(st, s->qkv, B, T, D, H, C, kc, vc, s->o)));
+        LAUNCH((launch_attn_prefill_mfma<WT, float>(st, s->qkv, B, T, D, H, C, kc, vc, s->o,
+                                                    s->ctx->props.multiProcessorCount)));
       else
         LAUNCH(launch_attn_prefill<WT>(st, s->qkv, B, T, D, H, C, kc, vc, s->o));
       FH_TRY(linear_parts<WT>(s, s->o, M, D, s->idx_blk(l, 4), D, &S));
@@ -595,7 +596,8 @@ int enqueue_layers_window(fh_session* s, int T, RowSrc src, LastRows* last) {
     LAUNCH(launch_kv_store<WT>(st, src, s->qkv, B, T, D, H, C, kc, vc));
     if (tail && l + 1 == s->d.n_layers) return enqueue_last_rows<WT, float>(s, T, src, l, s->qkv, 3 * D, last);
     if (D == 64 * H)
-      LAUNCH((launch_attn_prefill_mfma<WT, float>(st, s->qkv, B, T, D, H, C, kc, vc, s->o)));
+      LAUNCH((launch_attn_prefill_mfma<WT, float>(st, s->qkv, B, T, D, H, C, kc, vc, s->o,
+                                                  s->ctx->props.multiProcessorCount)));
     else
       LAUNCH(launch_attn_prefill<WT>(st, s->qkv, B, T, D, H, C, kc, vc, s->o));
     FH_TRY(linear<WT>(s, s->o, M, D, s->idx_blk(l, 4), D, s->v(s->idx_blk(l, 5)), EPI_NONE, s->x, s->x2));

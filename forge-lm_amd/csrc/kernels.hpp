@@ -81,7 +81,7 @@ hipError_t launch_attn_prefill(hipStream_t st, const float* qkv, int B, int T, i
 // bf16 (rounded) for a bf16 session's large-M GEMM.
 template <typename KT, typename OT>
 hipError_t launch_attn_prefill_mfma(hipStream_t st, const float* qkv, int B, int T, int d, int H, int ctx,
-                                    const KT* kcache, const KT* vcache, OT* o);
+                                    const KT* kcache, const KT* vcache, OT* o, int cus);
 
 // The same with q already in bf16, q [B*T][d] (from launch_gemm_bf16_qkv).
 hipError_t launch_attn_prefill_mfma_q16(hipStream_t st, const bf16_t* q, int B, int T, int d, int H, int ctx,

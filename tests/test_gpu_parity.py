@@ -1220,10 +1220,12 @@ def test_window_row_counts_match_oracle(fhp, oracle, backend, B, T):
         assert rel_err(got[b], rlg[0]) <= TOL_F32
 
 
-@pytest.mark.parametrize("B,T", [(1, 31), (1, 33), (2, 64), (1, 65), (1, 129), (3, 257), (130, 20), (65, 150)])
+@pytest.mark.parametrize("B,T", [(1, 31), (1, 32), (1, 33), (2, 64), (1, 65), (1, 97), (1, 129), (3, 257), (128, 40),
+                                 (129, 40), (64, 150), (65, 150)])
 def test_fp32_window_attention_blocks_match_oracle(fhp, oracle, backend, B, T):
-    """head_dim 64 windows in fp32 at the edges of the 32-query blocks and their 64-key tiles, with one to
-    five tiles over the four waves, and on both sides of the block count that picks 128-query blocks."""
+    """head_dim 64 windows in fp32 at the edges of the 32-query blocks and their 32-key tiles, with one to
+    nine tiles over the four waves, and on both sides of the two 128-query blocks per CU (512 on 256 CUs:
+    4 heads of 128 x 40 or 64 x 150 rows) that pick these."""
     m, oc, w = make_model(fhp, oracle, backend, (67, 300, 256, 2, 4), 5, batch=B)
     ids = np.stack([fhp.TrainingRandom(300 + b).ids(67, T) for b in range(B)])
     got = m.forward_last(ids)
