@@ -1089,7 +1089,11 @@ int ops_scratch(fh_context* c, OpsState* o, size_t bytes, void** p) {
     o->scratch = nullptr;
     o->scratch_bytes = 0;
     const size_t nb = std::max<size_t>(bytes, 1 << 16);
-    if (hipMalloc(&o->scratch, nb) != hipSuccess) return set_err(FH_ERR_OOM, "allocating %zu bytes of scratch", nb);
+    if (hipMalloc(&o->scratch, nb) != hipSuccess) {
+      o->scratch = nullptr;
+      (void)hipGetLastError();  // the next launch's check is its own
+      return set_err(FH_ERR_OOM, "allocating %zu bytes of scratch", nb);
+    }
     o->scratch_bytes = nb;
   }
   *p = o->scratch;
@@ -1164,9 +1168,13 @@ int matmul_common(fh_context* c, int mode, const void* a, const void* b, void* y
   const bool few = M < 1 << 22 && (K == 1 || (K <= 8 && (!acc || (size_t)M * N <= 1024)));
   if (!few && gemm_split_fits(slots, M, K, N)) {
     const int cus = context_cus(c);
-    const size_t pf = gemm_split_part_floats(slots, M, K, N, kSplitPartFloats, cus);
+    size_t pf = gemm_split_part_floats(slots, M, K, N, kSplitPartFloats, cus);
     void* part = nullptr;
-    if (pf) FH_TRY(ops_scratch(c, ops_, pf * sizeof(float), &part));
+    // a full device: K in one piece, which needs no scratch
+    if (pf && ops_scratch(c, ops_, pf * sizeof(float), &part) != FH_OK) {
+      part = nullptr;
+      pf = 0;
+    }
     HIP_TRY(launch_gemm_split(st_, mode, static_cast<const float*>(a), static_cast<const float*>(b), slots, M, K, N,
                               nullptr, 0, acc ? static_cast<const float*>(y) : nullptr, static_cast<float*>(y),
                               static_cast<float*>(part), pf, cus));
