@@ -497,7 +497,8 @@ __global__ __launch_bounds__(256) void k_ln_backward_dx(const float* __restrict_
 
 __global__ void k_ln_backward_cols(const float* __restrict__ dout, const float* __restrict__ x,
                                    const float* __restrict__ mean, const float* __restrict__ rstd, int rows, int cols,
-                                   int chunk_rows, float* __restrict__ part) {
+                                   int chunk_rows, float* __restrict__ dw, float* __restrict__ db,
+                                   float* __restrict__ part) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= cols) return;
   const int r0 = blockIdx.y * chunk_rows, r1 = min(rows, r0 + chunk_rows);
@@ -507,6 +508,11 @@ __global__ void k_ln_backward_cols(const float* __restrict__ dout, const float* 
     const float d = dout[(size_t)r * cols + c];
     s += d * ((x[(size_t)r * cols + c] - mean[r]) * rstd[r]);
     s2 += d;
+  }
+  if (!part) {  // all rows in one chunk
+    dw[c] = dw[c] + s;
+    db[c] = db[c] + s2;
+    return;
   }
   part[((size_t)blockIdx.y * 2) * cols + c] = s;
   part[((size_t)blockIdx.y * 2 + 1) * cols + c] = s2;
@@ -1393,20 +1399,21 @@ int fh_op_layernorm_backward(fh_context* c, const void* dout, const void* x, con
   const int per = wide ? std::max(32, (rows + 127) / 128) : std::max(4, ((rows + 511) / 512 + 3) / 4 * 4);
   const int chunks = (rows + per - 1) / per;
   void* p = nullptr;
-  FH_TRY(ops_scratch(c, ops_, (size_t)2 * chunks * cols * sizeof(float), &p));
+  if (!wide || chunks > 1) FH_TRY(ops_scratch(c, ops_, (size_t)2 * chunks * cols * sizeof(float), &p));
   float* part = static_cast<float*>(p);
   const float* fw = static_cast<const float*>(w);
-  float* fdx = static_cast<float*>(dx);
+  float *fdx = static_cast<float*>(dx), *fdw = static_cast<float*>(dw), *fdb = static_cast<float*>(db);
   if (wide) {
     hipLaunchKernelGGL(k_ln_backward_dx, dim3(rows), dim3(256), 0, st_, fd, fx, fw, fm, fr, fdx, cols);
     hipLaunchKernelGGL(k_ln_backward_cols, dim3((cols + 255) / 256, chunks), dim3(256), 0, st_, fd, fx, fm, fr, rows,
-                       cols, per, part);
+                       cols, per, fdw, fdb, part);
   } else {
     ROW_WAVES(k_ln_backward_rows, cols,
               <<<dim3(chunks), dim3(256), 0, st_>>>(fd, fx, fw, fm, fr, fdx, rows, cols, per, part));
   }
-  hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 63) / 64, 2), dim3(64 * kChunkWaves), 0, st_, part, chunks, cols,
-                     static_cast<float*>(dw), static_cast<float*>(db));
+  if (part)
+    hipLaunchKernelGGL(k_sum_chunks, dim3((cols + 63) / 64, 2), dim3(64 * kChunkWaves), 0, st_, part, chunks, cols, fdw,
+                       fdb);
   return op_launched("layernorm backward");
 }
 

@@ -891,7 +891,7 @@ def test_adamw_and_sum_squares_match_cpu(fhp, oracle, tb):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols", [(1, 1), (64, 63), (65, 64), (33, 65), (2049, 257), (700, 513), (2100, 769),
-                                       (5, 1024), (300, 1025)])
+                                       (5, 1024), (300, 1025), (1, 4001), (32, 2000), (33, 2000)])
 def test_column_reductions_chunks_and_widths(fhp, tb, rows, cols):
     """SumRows and LayerNormBackward (dx, dw, db) around their row chunks and row widths against
     float64.  A float32 sum of n terms in any order is off by at most n 2^-24 times the sum of their
