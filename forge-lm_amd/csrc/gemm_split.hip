@@ -35,11 +35,9 @@
 //
 // Small elements: bf16 ends at 2^-133 as fp32 does at 2^-149, so the three parts hold less than
 // 24 bits of an element below 2^-111 (sums of elements near 2^-118 came out 9e-6 off, near 2^-126
-// 2e-3).  What is lost is at most 2^-134 of the other
-// element, so it shows where the sum itself is tiny: a block with a sum below 2^-80 that is not
-// zero computes its tile again as well, which keeps fp32's precision for other elements up to
-// 2^29 / K^0.5.  The test costs 0.5-2% of a product of few stages (48 x 331 x 64 x 331: 16.3 ->
-// 16.6 us).
+// 2e-3).  What is lost is at most 2^-134 of the other element, so it shows where the sum itself is
+// tiny: a block with a sum below 2^-80 that is not zero computes its tile again as well, which keeps
+// fp32's precision for other elements up to 2^29 / K^0.5.
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -51,6 +49,7 @@ namespace {
 
 constexpr int SK = 32;  // k per stage: 64 bytes of bf16 per row and plane
 constexpr int FLIP = 2;  // stages between sign changes
+constexpr uint32_t kTiny = (127u - 80u) << 23;  // bits of 2^-80
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -199,7 +198,7 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   // The 64 x 64 tile has registers for a second accumulator: the five small products go there, so
   // the large sums are rounded K / 16 times and not 6 K / 16 (48 heads of 331 x 64: 3.4e-7 -> 1.4e-7
   // against 64 bits; windows of 33 to 128 rows at d 128: 2.6e-7 -> 1.8e-7, fp32 instructions 2.3e-7) at
-  // the same time.  128 x 64 would take 156 registers where it has 127: three blocks a CU, not four.
+  // the same time.  128 x 64 would take 156 registers where it has 128: three blocks a CU, not four.
   constexpr int NACC = MT * NT > 1 ? 1 : 2;
   __shared__ __align__(16) char smem[3 * (BM + BN) * 64];
   char* const As = smem;
@@ -325,21 +324,29 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   const int rows = min(BM, g.M - m0);
   const bool parts = g.part != nullptr;
   float* const out = parts ? g.part + (size_t)split * g.slots * g.M * g.N : g.y;
-  // rows and columns past the end may be flagged too: that costs time only
-  bool bad = false;
+  // the thread's place again, from a copy that the compiler takes for another value: kept in registers
+  // through the loop, what the rest derives from it displaced what the loop needs
+  int tid2 = threadIdx.x;
+  asm("" : "+v"(tid2));
+  const int lane2 = tid2 & 63, fr2 = lane2 & 31, fh2 = lane2 >> 5;
+  // rows and columns past the end may be flagged too: that costs time only.  Two instructions an
+  // element: a maximum that keeps NaN, and a minimum of the bits without sign, less one (0 wraps)
+  float most = 0.f;
+  uint32_t least = ~0u;
 #pragma unroll
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const float x = fabsf(acc[0][i][j][r]);
-        bad |= !(x < INFINITY) || (x < 0x1p-80f && x != 0.f);
+        most = __builtin_elementwise_maximum(most, fabsf(acc[0][i][j][r]));
+        least = min(least, (__float_as_uint(acc[0][i][j][r]) << 1) - 1);
       }
+  const bool bad = !(most < INFINITY) || least < 2 * kTiny - 1;
   if (__syncthreads_or(bad)) {
     // the tile again on the fp32 matrix cores, which give what fp32 arithmetic gives
-    oa.init(a, AKC ? g.K : g.M, g.M, m0, g.K, kb, tid);
-    ob.init(b, BKC ? g.K : g.N, g.N, n0, g.K, kb, tid);
+    oa.init(a, AKC ? g.K : g.M, g.M, m0, g.K, kb, tid2);
+    ob.init(b, BKC ? g.K : g.N, g.N, n0, g.K, kb, tid2);
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -359,11 +366,12 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
       oa.store_f32(As, va);
       ob.store_f32(As + BM * 128, vb);
       __syncthreads();
-      // a step's two k are k and k + 16 of the stage: 16 bytes of a row feed four steps
-#pragma unroll
+      // a step's two k are k and k + 16 of the stage: 16 bytes of a row feed four steps.  (Unrolled, these
+      // steps cost the loop above registers: 768 x 2048 x 3072 TN 74.9 -> 76.9 us.)
+#pragma unroll 1
       for (int kk = 0; kk < SK / 8; kk++) {
         float4 af[MT], bf[NT];
-        const int at = fr * 128 + 16 * ((4 * fh + kk) ^ (fr & 7));
+        const int at = fr2 * 128 + 16 * ((4 * fh2 + kk) ^ (fr2 & 7));
 #pragma unroll
         for (int i = 0; i < MT; i++)
           af[i] = *reinterpret_cast<const float4*>(As + (wm * (BM / 2) + i * 32) * 128 + at);
@@ -390,20 +398,20 @@ __global__ __launch_bounds__(256, 3) void k_gemm_split(SplitArgs g) {
   const __amdgpu_buffer_rsrc_t rres = !parts && g.res ? rows_rsrc(g.res, yrow, rows, g.N, 4) : ry;
 #pragma unroll
   for (int j = 0; j < NT; j++) {
-    const int col = n0 + wn * (BN / 2) + j * 32 + fr;
+    const int col = n0 + wn * (BN / 2) + j * 32 + fr2;
     if (col >= g.N) continue;
     const float bcol = !parts && g.bias ? g.bias[col] : 0.f;
 #pragma unroll
     for (int i = 0; i < MT; i++) {
       const int tr = wm * (BM / 2) + i * 32;
       if (parts)
-        mfma_store_tile<EPI_NONE, false, false, 2>(acc[0][i][j], lane, tr, col, g.N, 0.f, ry, ry);
+        mfma_store_tile<EPI_NONE, false, false, 2>(acc[0][i][j], lane2, tr, col, g.N, 0.f, ry, ry);
       else if (g.gelu)
-        mfma_store_tile<EPI_GELU, false, false>(acc[0][i][j], lane, tr, col, g.N, bcol, ry, ry);
+        mfma_store_tile<EPI_GELU, false, false>(acc[0][i][j], lane2, tr, col, g.N, bcol, ry, ry);
       else if (g.res)
-        mfma_store_tile<EPI_NONE, true, false>(acc[0][i][j], lane, tr, col, g.N, bcol, rres, ry);
+        mfma_store_tile<EPI_NONE, true, false>(acc[0][i][j], lane2, tr, col, g.N, bcol, rres, ry);
       else
-        mfma_store_tile<EPI_NONE, false, false>(acc[0][i][j], lane, tr, col, g.N, bcol, ry, ry);
+        mfma_store_tile<EPI_NONE, false, false>(acc[0][i][j], lane2, tr, col, g.N, bcol, ry, ry);
     }
   }
 }
