@@ -449,8 +449,8 @@ size_t split_blocks(int bm, int bn, int slots, int M, int N) {
 // `round` more per round of blocks over the CUs; a stage costs a CU `unit` per block of its own
 // (a large tile does the most per operand byte: 217 / 190 / 168 TFLOP/s at 8192 x 4096 x 4096),
 // a lone block no less than `alone` (its chain of load, split, LDS and MFMAs); splitting K costs a
-// second launch and the partial sums' way through memory.  2048 x 3072 x 768: 128 x 128 tiles in
-// 8 splits 64 us, unsplit 109; 100 x 768 x 768: 64 x 64 in 8 splits 9.5, unsplit 23.
+// second launch and the partial sums' way through memory.  M 2048, K 3072, N 768: 128 x 128 tiles in
+// 5 splits, 72 us with their sum, unsplit 109; 100 x 768 x 768: 64 x 64 in 12 splits, 11.3, unsplit 23.
 SplitPlan split_plan(int slots, int M, int K, int N, size_t part_floats, int cus) {
   constexpr double fixed[3] = {4.6, 3.9, 4.1}, round[3] = {1.5, 0.7, 0.24};
   constexpr double alone[3] = {1.78, 1.2, 0.77}, unit[3] = {1.17, 0.74, 0.45};

@@ -10,10 +10,11 @@
 // contract (InvalidateDeviceCache / EnsureHostCurrent) lives in the host
 // mirror, which owns the device copies of its tensors.
 //
-// The kernels are the straightforward HBM-bound forms: grid-stride elementwise
-// loops, one block or wave per row for the row reductions, column sums in chunks of rows
-// in a fixed order; the (batched) matmuls run on the split GEMM (gemm_split.hip).
-// Results follow CpuBackend
+// Elementwise kernels move 16 bytes to a load where the pointers allow it; rows of up to 1024 columns
+// (softmax, LayerNorm, cross-entropy) stay in a wave's registers, of up to 32768 (cross-entropy) in
+// a block's, wider ones take a block and several passes; column sums go by chunks of rows in a fixed
+// order; the (batched) matmuls run on the split GEMM (gemm_split.hip), those of few k or of sizes
+// past it on the tiled kernel here.  Results follow CpuBackend
 // within the reference's own GPU-contract tolerances (GpuBackendTests.cs:23-24:
 // 1e-4 forward, 1e-2 backward); the gathers, copies, masks and the embedding
 // scatter-add (which adds each index's rows in ascending position, as the CPU
