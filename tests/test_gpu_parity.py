@@ -1286,3 +1286,22 @@ def test_batched_decode_splits_match_oracle(fhp, oracle, backend, B):
     for b in (0, B - 1):
         rids, rlg = oracle.generate(oc, w, prompts[b], 4, return_logits=True)
         assert_greedy_parity(ids[b], lg[b], rids, rlg, TOL_F32, f"sequence {b}")
+
+
+@pytest.mark.parametrize("T", [33, 100, 1000])
+def test_fp32_windows_of_tiny_weights_match_oracle(fhp, oracle, backend, T):
+    """Blocks whose matrices are 1e-30 of their size: every product of the window is computed again in fp32 and its
+    bias, GELU, residual or partial sums come after that."""
+    shape = (67, 1000, 128, 2, 2)
+    m, oc, w = make_model(fhp, oracle, backend, shape, 3)
+    o = 0
+    for name, n in fhp.registry(fhp.ModelConfig(*shape)):
+        if name.startswith("blocks.") and name.endswith((".qkv.w", ".proj.w", ".fc.w")):
+            w[o:o + n] *= 1e-30
+        o += n
+    m.load_weights(w)
+    ids = fhp.TrainingRandom(7).ids(67, T)
+    got = m.forward_last(ids)
+    m.dispose()
+    _, rlg = oracle.generate(oc, w, ids, 1, return_logits=True)
+    assert rel_err(got[0], rlg[0]) <= TOL_F32
